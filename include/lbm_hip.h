@@ -79,6 +79,18 @@
  *                     8-byte accesses (auto, default; the list kernel only
  *                     when the padded node count allows), or one per
  *                     thread (1)
+ *   -two-step auto|on|off
+ *                     an even and an odd step in one launch, from the PDF
+ *                     array into a second one, with the same results (auto,
+ *                     default: on lattices where it measured faster, unless
+ *                     an option of the separate launches -- -bs, -adj, -nt,
+ *                     -even-cap, -odd-order, -even-order, -odd-pairs, -vec --
+ *                     is given; on: wherever the faces allow it; off).  The
+ *                     second array (aa-soa: two) and an index map are taken
+ *                     at the first Kernel() call (aa-soa: at Init), only
+ *                     where they fit into half of the free device memory;
+ *                     otherwise, with -launch-events, with a non-finite body
+ *                     force and in a batch the steps are launched one by one
  *   -odd-pairs auto|on|off
  *                     aa-soa at fp32s with -vec auto: the odd step takes
  *                     pairs of z cells, one access per direction for a pair
@@ -291,8 +303,8 @@ int LbmHipBatchGraphStats(LbmHipBatch * b, int * slots, long long * captures, lo
  * the lattice ld with these kernel arguments (padding, storage type, ...),
  * computed on the host without touching the device: every allocation
  * Init makes, its temporary buffers included, the run-compressed adjacency
- * at its largest, each rounded up to 2 MiB.  For admission against a
- * memory budget (the serving loop). */
+ * at its largest, each rounded up to 2 MiB.  What Kernel() takes for -two-step
+ * is not in it.  For admission against a memory budget (the serving loop). */
 int LbmHipListDeviceBytes(const LatticeDesc * ld, const Parameters * params, uint64_t * bytes);
 
 /* Copies the device list build to caller buffers, in the reference's

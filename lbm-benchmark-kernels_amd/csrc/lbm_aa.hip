@@ -41,10 +41,13 @@ void VtkWrite(LatticeDesc * ld, KernelData * kd, CaseData * cd, int iteration) _
 void KernelStatistics(KernelData * kd, LatticeDesc * ld, CaseData * cd, int iteration) __attribute__((weak));
 }
 
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 #include <new>
+#include <type_traits>
+#include <utility>
 
 namespace lbm {
 
@@ -73,6 +76,7 @@ struct AaData {
 	void * hPdf = nullptr;
 	uint32_t * hInfo = nullptr;
 	size_t nPdf = 0;
+	PairPlan pair;                // even and odd step in one launch, on dense copies of the fluid cells' values
 	double * dMoments = nullptr;  // per-block pairs, then the total (allocated at first use)
 	uint32_t momentBlocks = 0;
 	// run-time output after an even step: GetNode serves the reference's
@@ -148,6 +152,60 @@ __global__ __launch_bounds__(256) void k_aa_fluid_bits(const uint32_t * __restri
 	for (int j = 0; j < 64 && z0 + j < g.Z; ++j)
 		if (info[row * (uint64_t)g.Z + z0 + j] & kInfoFluid) w |= 1ull << j;
 	bits[i] = w;
+}
+
+// Fluid cells of every z row, [x][y].
+__global__ __launch_bounds__(256) void k_aa_row_counts(const unsigned long long * __restrict__ bits, AaGeom g,
+                                                       uint32_t * __restrict__ count)
+{
+	const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+	if (r >= (uint32_t)g.X * g.Y) return;
+	uint32_t n = 0;
+	for (int w = 0; w < g.zWords; ++w) n += (uint32_t)__popcll(bits[(size_t)r * g.zWords + w]);
+	count[r] = n;
+}
+
+// The cell map of the two-step launch (PairPlan.map), z fastest, with the x
+// ghost planes: the number of every fluid cell in this order (rowBase: fluid
+// cells before each z row) plus one.
+__global__ __launch_bounds__(256) void k_aa_pair_map(const unsigned long long * __restrict__ bits, AaGeom g,
+                                                     const uint32_t * __restrict__ rowBase, uint32_t * __restrict__ map)
+{
+	const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+	if (i >= (uint64_t)(g.X + 2) * g.Y * g.Z) return;
+	const int z = (int)(i % (uint64_t)g.Z), y = (int)(i / (uint64_t)g.Z % (uint64_t)g.Y);
+	int x = (int)(i / ((uint64_t)g.Z * g.Y)) - 1;
+	if (x < 0 || x >= g.X) x = !g.px ? -1 : x < 0 ? g.X - 1 : 0;
+	uint32_t id = 0;
+	if (x >= 0) {
+		const unsigned long long * row = bits + ((size_t)x * g.Y + y) * g.zWords;
+		if ((row[z >> 6] >> (z & 63)) & 1ull) {
+			id = rowBase[(size_t)x * g.Y + y] + 1u;
+			for (int w = 0; w < z >> 6; ++w) id += (uint32_t)__popcll(row[w]);
+			id += (uint32_t)__popcll(row[z >> 6] & ((1ull << (z & 63)) - 1ull));
+		}
+	}
+	map[i] = id;
+}
+
+// The fluid cells' values between the full array and the dense one of the
+// two-step launch (DENSE: into the dense one).  Both are streamed once.
+template <class S, bool DENSE>
+__global__ __launch_bounds__(256) void k_aa_dense(S * __restrict__ pdf, S * __restrict__ dense,
+                                                  const uint32_t * __restrict__ map, AaGeom g, uint64_t plane)
+{
+	const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+	if (i >= (uint32_t)g.X * g.Y * g.Z) return;
+	const uint32_t id = map[(size_t)g.Y * g.Z + i];          // behind the ghost plane
+	if (id == 0) return;
+	const int z = (int)(i % (uint32_t)g.Z), y = (int)(i / (uint32_t)g.Z % (uint32_t)g.Y), x = (int)(i / ((uint32_t)g.Z * g.Y));
+	S * a = pdf + aa_slot(g, 0, x, y, z);
+	S * b = dense + (id - 1u);
+#pragma unroll
+	for (int d = 0; d < 19; ++d) {
+		if (DENSE) b[(size_t)d * plane] = a[(size_t)d * g.plane];
+		else       a[(size_t)d * g.plane] = b[(size_t)d * plane];
+	}
 }
 
 __device__ __forceinline__ unsigned long long aa_fluid_word(const unsigned long long * bits, const AaGeom & g, int x, int y,
@@ -639,10 +697,45 @@ static bool aa_upload(AaData * A)
 	if (!c.shadowDirty) { c.t.uploadMs = 0.0; return true; }
 	const double t0 = (double)clock() / CLOCKS_PER_SEC;
 	if (!hip_ok(hipMemcpyAsync(A->dPdf, A->hPdf, aa_bytes(A), hipMemcpyHostToDevice, c.stream), "upload of the host lattice")) return false;
+	A->pair.current = false;
 	if (!hip_ok(hipStreamSynchronize(c.stream), "hipStreamSynchronize")) return false;
 	c.t.uploadMs = ((double)clock() / CLOCKS_PER_SEC - t0) * 1e3;
 	c.shadowDirty = 0;
 	return true;
+}
+
+// The fluid cells' values into the dense array of the two-step launch, or
+// back from it.
+static void aa_dense_copy(AaData * A, bool toDense)
+{
+	const AaGeom & g = A->g;
+	const unsigned nb = (unsigned)(((uint64_t)g.X * g.Y * g.Z + 255) / 256);
+	auto launch = [&](auto * pdf) {
+		using S = std::remove_pointer_t<decltype(pdf)>;
+		if (toDense) k_aa_dense<S, true><<<nb, 256, 0, A->c.stream>>>(pdf, (S *)A->pair.dense, A->pair.map, g, A->pair.plane);
+		else         k_aa_dense<S, false><<<nb, 256, 0, A->c.stream>>>(pdf, (S *)A->pair.dense, A->pair.map, g, A->pair.plane);
+	};
+	switch (A->c.args.prec) {
+		case PREC_FP32S: launch((float *)A->dPdf); break;
+		case PREC_FP16S: launch((uint16_t *)A->dPdf); break;
+		default: launch((double *)A->dPdf);
+	}
+	A->pair.current = true;
+}
+
+// The arrays of the two-step launch; the number of fluid cells in the mask to
+// *count (device).
+static void aa_build_pair(AaData * A, const LatticeDesc * ld, uint32_t * count, hipStream_t s)
+{
+	const AaGeom & g = A->g;
+	PairPlan & p = A->pair;
+	pair_plan(&p, A->c.args, A->c.nCU, ld, 0, false);
+	pair_alloc(&p);
+	if (!p.use) return;
+	const uint32_t rows = (uint32_t)g.X * g.Y;
+	k_aa_row_counts<<<(rows + 255) / 256, 256, 0, s>>>(A->dFluid, g, p.rows);
+	scan_exclusive(p.rows, rows, count, s);
+	k_aa_pair_map<<<(unsigned)((pair_map_cells(p) + 255) / 256), 256, 0, s>>>(A->dFluid, g, p.rows, p.map);
 }
 
 // Host copy of the current state for the output functions' GetNode.
@@ -757,6 +850,7 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 	                    A->dFluid, g, nt};
 	const float f16s = (float)(1 << c.args.f16Shift);
 	auto half = [&](bool on, bool fl, bool fs, int it, bool doEven, bool doOdd) {
+		A->pair.current = false;
 		hipEvent_t * ev = perLaunch ? c.ev + 2 * it : nullptr;
 		switch (c.args.prec) {
 			case PREC_FP32S: aa_launch(L, (float *)A->dPdf, CodecF32{}, k, ft, on, fl, fs, ev, doEven, doOdd); break;
@@ -773,6 +867,21 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 		return aa_download(kd);
 	};
 
+	// both steps in one launch; per-launch timing needs two, and an infinite
+	// or NaN force (whose zero components are NaN) the full force table
+	const bool pairs = A->pair.use && !perLaunch && isfinite(cd->XForce);
+	bool inDense = false;      // the dense array is ahead of the full one
+	auto pair = [&](bool fl, bool fs) {
+		if (!A->pair.current) aa_dense_copy(A, true);
+		pair_launch(A->pair, A->pair.dense, A->pair.other, k, ft, fl, force, fs, c.stream);
+		std::swap(A->pair.dense, A->pair.other);
+		inDense = true;
+	};
+	// the full array up to date again, for whatever reads it next
+	auto pairs_done = [&]() {
+		if (inDense) aa_dense_copy(A, false);
+		inDense = false;
+	};
 	(void)hipGetLastError();   // launch checks below must see only this loop's errors
 	if (!hip_ok(hipEventRecord(c.evLoop[0], c.stream), "hipEventRecord")) return false;
 	bool segmentStart = true;  // the force of the previous step is in the stored values
@@ -781,9 +890,16 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 	if (useGraph) {
 		// the same launches as the loop below without output, replayed
 		auto record = [&]() {
-			for (int it = 0; it < steps; it += 2) half(force, force && it > 0, force && it + 2 >= steps, it, true, true);
+			for (int it = 0; it < steps; it += 2) {
+				const bool fl = force && it > 0, fs = force && it + 2 >= steps;
+				if (pairs) pair(fl, fs);
+				else half(force, fl, fs, it, true, true);
+			}
+			pairs_done();
 		};
-		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, record)) return false;
+		A->pair.current = false;   // every replay begins and ends with the full array
+		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, A->dPdf, record)) return false;
+		A->pair.current = false;
 		synced = false;
 	}
 	for (int it = 0; it < steps && A->nFluid > 0 && !useGraph; it += 2) {
@@ -792,9 +908,12 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 		const bool mid = statsEven || vtkEven, end = vtkOdd || statsOdd;
 		const bool last = it + 2 >= steps || end;
 		synced = false;
-		if (!mid) {
+		if (!mid && pairs) {
+			pair(force && !segmentStart, force && last);
+		} else if (!mid) {
 			half(force, force && !segmentStart, force && last, it, true, true);
 		} else {
+			pairs_done();
 			half(force, force && !segmentStart, false, it, true, false);
 			if (!output_state()) return false;
 			c.iteration = it - 1;              // before the fix-ups: the swapped values in the local view
@@ -809,6 +928,7 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 		}
 		segmentStart = last;
 		if (end) {
+			pairs_done();
 			if (!output_state()) return false;
 			synced = true;
 			c.iteration = it + 1;
@@ -816,6 +936,7 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 			if (statsOdd) KernelStatistics(kd, ld, ccd, it + 1);
 		}
 	}
+	pairs_done();
 	if (!hip_ok(hipGetLastError(), "step kernel launch")) return false;
 	if (!hip_ok(hipEventRecord(c.evLoop[1], c.stream), "hipEventRecord")) return false;
 	if (!hip_ok(hipStreamSynchronize(c.stream), "step kernels")) return false;
@@ -903,6 +1024,7 @@ static void aa_release(AaData * A)
 	(void)hipFree(A->dInfo);
 	(void)hipFree(A->dFluid);
 	(void)hipFree(A->dPdf);
+	pair_free(&A->pair);
 	host_free(A->hPdf);
 	free(A->hInfo);
 	common_free(&A->c);
@@ -973,23 +1095,24 @@ void D3Q19AaInit_AaSoAHip(LatticeDesc * ld, KernelData ** kernelData, Parameters
 
 	int * dMask = nullptr;
 	uint32_t * dCount = nullptr;
-	uint32_t hCount = 0;
+	uint32_t hCount[2] = {0, 0};     // bounce-back pairs; fluid cells (with a two-step plan)
 	bool ok = false;
 	hipStream_t s = A->c.stream;
 	do {
 		if (!hip_ok(hipMalloc((void **)&dMask, sizeof(int) * nTotal), "allocating geometry mask")) break;
-		if (!hip_ok(hipMalloc((void **)&dCount, sizeof(uint32_t)), "allocating counter")) break;
+		if (!hip_ok(hipMalloc((void **)&dCount, sizeof(hCount)), "allocating counter")) break;
 		if (!hip_ok(hipMalloc((void **)&A->dInfo, sizeof(uint32_t) * nTotal), "allocating cell info")) break;
 		const uint64_t nWords = (uint64_t)g.X * g.Y * g.zWords;
 		if (!hip_ok(hipMalloc((void **)&A->dFluid, sizeof(unsigned long long) * nWords), "allocating fluid mask")) break;
 		if (!hip_ok(hipMalloc((void **)&A->dPdf, aa_bytes(A)), "allocating device lattice")) break;
 		if (!hip_ok(hipMemcpyAsync(dMask, ld->Lattice, sizeof(int) * nTotal, hipMemcpyHostToDevice, s), "mask upload")) break;
-		if (!hip_ok(hipMemsetAsync(dCount, 0, sizeof(uint32_t), s), "hipMemset")) break;
+		if (!hip_ok(hipMemsetAsync(dCount, 0, sizeof(hCount), s), "hipMemset")) break;
 		(void)hipGetLastError();
 		k_aa_info<<<(unsigned)((nTotal + 255) / 256), 256, 0, s>>>(dMask, g, A->dInfo, dCount);
 		k_aa_fluid_bits<<<(unsigned)((nWords + 255) / 256), 256, 0, s>>>(A->dInfo, g, A->dFluid);
+		aa_build_pair(A, ld, dCount + 1, s);
 		if (!hip_ok(hipGetLastError(), "cell info kernel")) break;
-		if (!hip_ok(hipMemcpyAsync(&hCount, dCount, sizeof(uint32_t), hipMemcpyDeviceToHost, s), "count download")) break;
+		if (!hip_ok(hipMemcpyAsync(hCount, dCount, sizeof(hCount), hipMemcpyDeviceToHost, s), "count download")) break;
 		A->hPdf = host_alloc(aa_bytes(A));
 		if (!A->hPdf) { fail("allocating host lattice failed: %zu bytes.", aa_bytes(A)); break; }
 		// every slot starts as f = 0, ghost cells included; shifted storage
@@ -1007,8 +1130,13 @@ void D3Q19AaInit_AaSoAHip(LatticeDesc * ld, KernelData ** kernelData, Parameters
 	(void)hipFree(dMask);
 	(void)hipFree(dCount);
 	if (!ok) { aa_release(A); return; }
-	A->nBounce = (int)hCount;
-	if (!A->c.args.quiet) printf("# bounce back pdfs: %d (resolved in the odd step, no index lists)\n", A->nBounce);
+	A->nBounce = (int)hCount[0];
+	// the dense planes are sized by nFluid
+	if (A->pair.use && hCount[1] != (uint32_t)A->nFluid) pair_free(&A->pair);
+	if (!A->c.args.quiet) {
+		pair_report(A->pair);
+		printf("# bounce back pdfs: %d (resolved in the odd step, no index lists)\n", A->nBounce);
+	}
 
 	KernelData * kd = &A->kd;
 	kd->Pdfs[0] = (PdfT *)A->hPdf;     // storage type given by -prec (double by default)

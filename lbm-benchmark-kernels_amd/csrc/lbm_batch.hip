@@ -789,6 +789,8 @@ LbmHipBatch * LbmHipBatchCreate(const Parameters * params)
 	b->words.emplace_back("lazy");
 	for (int i = 0; i < n; ++i) b->words.emplace_back(params->KernelArgs[i]);
 	b->words.emplace_back("-quiet");
+	b->words.emplace_back("-two-step");      // the batch's own launches step the domains
+	b->words.emplace_back("off");
 	for (std::string & w : b->words) b->argv.push_back(&w[0]);
 	b->params.nKernelArgs = (int)b->argv.size();
 	b->params.KernelArgs = b->argv.data();

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "lbm_device.h"
+#include "lbm_pair.h"
 #include "lbm_runtime.h"
 
 namespace lbm {
@@ -26,7 +27,9 @@ struct ListData {
 	uint32_t * dGrid = nullptr;
 	uint32_t * dCoords = nullptr;
 	uint32_t * dAdj = nullptr;
-	void * dPdf = nullptr;       // 19 * nCells values of the storage type
+	void * dPdf = nullptr;       // 19 * nCells values of the storage type: dPdfOwn or pair.other
+	void * dPdfOwn = nullptr;
+	PairPlan pair;               // even and odd step in one launch; a launch swaps dPdf and pair.other
 	void * hPdf = nullptr;       // host shadow, same layout and type, == kd.Pdfs[0]
 	double * dMoments = nullptr; // reduction scratch: 2 per block + 2
 	uint32_t * dOddOrder = nullptr; // odd step, -odd-order band: node block of each launched block
@@ -42,6 +45,8 @@ ListData * list_data(KernelData * kd);
 // Host shadow -> device when SetNode touched it; device -> host shadow.
 bool list_upload(ListData * L);
 bool list_download(ListData * L);
+// Exclusive prefix sum of n device words in place, the total to *sum.
+void scan_exclusive(uint32_t * v, uint32_t n, uint32_t * sum, hipStream_t stream);
 // Bytes of one stored value for a -prec setting.
 size_t elem_bytes(int prec);
 

@@ -34,11 +34,13 @@ void VtkWrite(LatticeDesc * ld, KernelData * kd, CaseData * cd, int iteration) _
 void KernelStatistics(KernelData * kd, LatticeDesc * ld, CaseData * cd, int iteration) __attribute__((weak));
 }
 
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 #include <mutex>
 #include <new>
+#include <utility>
 #include <vector>
 
 namespace lbm {
@@ -127,6 +129,11 @@ __global__ __launch_bounds__(1024) void k_scan_once(uint32_t * __restrict__ v, u
 		run += c;
 	}
 	if (tid == 1023) *sum = part[1023];
+}
+
+void scan_exclusive(uint32_t * v, uint32_t n, uint32_t * sum, hipStream_t stream)
+{
+	k_scan_once<<<1, 1024, 0, stream>>>(v, n, sum);
 }
 
 __global__ __launch_bounds__(kNumBlock) void k_num_assign(const int * __restrict__ mask, NumGeom g, uint32_t N,
@@ -438,6 +445,34 @@ static void list_bc_set(KernelData * kd, int x, int y, int z, int dir, PdfT pdf)
 	L->c.shadowDirty = 1;
 }
 
+// The cell map of the two-step launch (PairPlan.map) from the grid of node
+// ids: index + 1 of every cell, z fastest, with the x ghost planes.
+__global__ __launch_bounds__(256) void k_list_pair_map(const uint32_t * __restrict__ grid, int X, int Y, int Z, int px,
+                                                       uint32_t * __restrict__ map)
+{
+	const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+	if (i >= (uint64_t)(X + 2) * Y * Z) return;
+	const int z = (int)(i % (uint64_t)Z), y = (int)(i / (uint64_t)Z % (uint64_t)Y);
+	int x = (int)(i / ((uint64_t)Z * Y)) - 1;
+	if (x < 0 || x >= X) x = !px ? -1 : x < 0 ? X - 1 : 0;
+	map[i] = x < 0 ? 0u : grid[((size_t)z * Y + y) * X + x] + 1u;   // no node: 0xffffffff + 1
+}
+
+// The second PDF array and the cell map of the two-step launch, made at the
+// first call that can use them: Init takes no more device memory than
+// LbmHipListDeviceBytes states, and a lattice that a batch steps needs none.
+static bool list_build_pair(ListData * L)
+{
+	if (!L->pair.use || L->pair.block) return true;
+	pair_alloc(&L->pair);
+	if (!L->pair.use) return true;
+	(void)hipGetLastError();
+	k_list_pair_map<<<(unsigned)((pair_map_cells(L->pair) + 255) / 256), 256, 0, L->c.stream>>>(
+		L->dGrid, L->dims[0], L->dims[1], L->dims[2], L->periodic[0], L->pair.map);
+	return hip_ok(hipGetLastError(), "cell map kernel") &&
+	       hip_ok(hipMemsetAsync(L->pair.other, 0, elem_bytes(L->c.args.prec) * 19 * (size_t)L->nCells, L->c.stream), "hipMemset");
+}
+
 // ------------------------------------------------------------- Kernel()
 // The fluid nodes' values between the device lattice and its host copy, 19
 // rows of the planes: the padding (up to 264208 nodes a plane for the smallest
@@ -671,34 +706,54 @@ static bool list_steps(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 			default:         launch_odd(cfg, (double *)L->dPdf, CodecF64{}, full, runs, k, ft, fl, fs);
 		}
 	};
+	// both steps in one launch; per-launch timing needs two, and an infinite
+	// or NaN force (whose zero components are NaN) the full force table
+	bool pairs = L->pair.use && !perLaunch && isfinite(cd->XForce) && steps > 0;
+	if (pairs && !list_build_pair(L)) return false;
+	pairs = pairs && L->pair.use;
+	auto pair = [&](bool fl, bool fs) {
+		pair_launch(L->pair, L->dPdf, L->pair.other, k, ft, fl, force, fs, c.stream);
+		std::swap(L->dPdf, L->pair.other);
+	};
 	(void)hipGetLastError();   // launch checks below must see only this loop's errors
 	if (!hip_ok(hipEventRecord(c.evLoop[0], c.stream), "hipEventRecord")) return false;
 	bool segmentStart = true;  // the force of the previous step is in the stored values
 	bool synced = true;        // the host copy holds the state of the last launch
 	const bool useGraph = c.args.graph && !perLaunch && !out.vtk && !out.stats && steps > 0 && L->nFluid > 0;
 	if (useGraph) {
-		// the same launches as the loop below without output, replayed
+		// the same launches as the loop below without output, replayed; an odd
+		// number of pairs begins with one in place, so that a replay ends in
+		// the array it began with
 		auto record = [&]() {
 			for (int it = 0; it < steps; it += 2) {
-				even(force && it > 0);
-				odd(force, force && it + 2 >= steps);
+				const bool fl = force && it > 0, fs = force && it + 2 >= steps;
+				if (pairs && !(it == 0 && steps % 4)) {
+					pair(fl, fs);
+				} else {
+					even(fl);
+					odd(force, fs);
+				}
 			}
 		};
-		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, record)) return false;
+		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, L->dPdf, record)) return false;
 		synced = false;
 	}
 	for (int it = 0; it < steps && L->nFluid > 0 && !useGraph; it += 2) {
 		const bool output = out.at(cd, it);
 		synced = false;
 		const bool last = it + 2 >= steps || output;
-		if (perLaunch) (void)hipEventRecord(c.ev[2 * it], c.stream);
-		even(force && !segmentStart);
-		if (perLaunch) {
-			(void)hipEventRecord(c.ev[2 * it + 1], c.stream);
-			(void)hipEventRecord(c.ev[2 * it + 2], c.stream);
+		if (pairs) {
+			pair(force && !segmentStart, force && last);
+		} else {
+			if (perLaunch) (void)hipEventRecord(c.ev[2 * it], c.stream);
+			even(force && !segmentStart);
+			if (perLaunch) {
+				(void)hipEventRecord(c.ev[2 * it + 1], c.stream);
+				(void)hipEventRecord(c.ev[2 * it + 2], c.stream);
+			}
+			odd(force, force && last);
+			if (perLaunch) (void)hipEventRecord(c.ev[2 * it + 3], c.stream);
 		}
-		odd(force, force && last);
-		if (perLaunch) (void)hipEventRecord(c.ev[2 * it + 3], c.stream);
 		segmentStart = last;
 		if (output) {
 			if (!hip_ok(hipGetLastError(), "step kernel launch")) return false;
@@ -781,8 +836,9 @@ static void list_release(ListData * L)
 	(void)hipFree(L->dRunMask);
 	(void)hipFree(L->dRunBase);
 	(void)hipFree(L->dRunAdj);
-	(void)hipFree(L->dPdf);
+	(void)hipFree(L->dPdfOwn);
 	(void)hipFree(L->dMoments);
+	pair_free(&L->pair);
 	host_free(L->hPdf);
 	free(L->hGrid);
 	common_free(&L->c);
@@ -991,8 +1047,10 @@ void D3Q19ListAaPvInit_PushSoAHip(LatticeDesc * ld, KernelData ** kernelData, Pa
 	// f = w, for FP64 f = 0 as the reference initialises
 	// (src/BenchKernelD3Q19ListAaPvCommon.c:583-585)
 	const size_t pdfBytes = elem_bytes(L->c.args.prec) * 19 * (size_t)L->nCells;
-	if (!dev_alloc((void **)&L->dPdf, pdfBytes, "device lattice")) { list_release(L); return; }
+	if (!dev_alloc((void **)&L->dPdfOwn, pdfBytes, "device lattice")) { list_release(L); return; }
+	L->dPdf = L->dPdfOwn;
 	if (!hip_ok(hipMemsetAsync(L->dPdf, 0, pdfBytes, L->c.stream), "hipMemset")) { list_release(L); return; }
+	pair_plan(&L->pair, L->c.args, L->c.nCU, ld, (uint64_t)L->nCells, true);
 	L->momentBlocks = (L->nFluid + 255) / 256;
 	if (!dev_alloc((void **)&L->dMoments, sizeof(double) * (2 * (size_t)L->momentBlocks + 2), "moment scratch")) { list_release(L); return; }
 	if (!L->c.args.lazyShadow) {
@@ -1006,6 +1064,7 @@ void D3Q19ListAaPvInit_PushSoAHip(LatticeDesc * ld, KernelData ** kernelData, Pa
 	if (!L->c.args.quiet) {
 		printf("# total fluid nodes: %d   consecutive blocks: %d   runs cut at wavefronts: %d\n",
 		       L->nFluid, L->nRuns, L->nRunsWave);
+		pair_report(L->pair);
 		printf("# loop balance:          %.2f B/FLUP  even: %.2f B/FLUP  odd %.2f B/FLUP\n", (even + odd) / 2, even, odd);
 	}
 

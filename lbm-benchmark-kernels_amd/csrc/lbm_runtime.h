@@ -54,6 +54,9 @@ struct KernelArgs {
 	int statistics = 0;    // list: KernelStatistics during the run (the reference's STATISTICS build)
 	int oddOrder = 2;      // list: odd-step block order, 0 plain, 1 XCD-grouped, 2 y bands per XCD
 	int evenDown = 0;      // list: even step in descending block order (starts where the odd step ended)
+	int twoStep = -1;      // even and odd step of a single lattice in one launch: 1 where possible, 0 never,
+	                       // -1 where it measured faster and no option of the separate launches was given
+	int splitOption = 0;   // an option of the separate even / odd launches was given
 	int launchEvents = 0;  // per-launch timing events (even/odd averages)
 	int graph = 0;         // replay the step loop of a Kernel() call from a captured HIP graph
 };
@@ -121,6 +124,7 @@ struct Common {
 	hipGraphExec_t graphExec = nullptr;
 	int graphSteps = 0;
 	double graphOmega = 0.0, graphForce = 0.0;
+	const void * graphPdf = nullptr;
 };
 
 // SetNode may change the host shadow only while it holds the device's
@@ -151,14 +155,15 @@ bool common_events(Common * c, int launches);
 // Fills c->t from the recorded events (stream must be synchronised).
 void common_collect(Common * c, int launches, bool perLaunch);
 
-// Runs the step loop of `steps` steps for (omega, xForce) on c->stream by
-// replaying a HIP graph; `record` issues the loop's kernel launches and is
+// Runs the step loop of `steps` steps for (omega, xForce) on the lattice at
+// `pdf` on c->stream by replaying a HIP graph; `record` issues the loop's kernel launches and is
 // called, under stream capture, only when no graph was captured for these
 // values yet.  The graph holds kernel launches only.
 template <class F>
-bool common_graph_run(Common * c, int steps, double omega, double xForce, F record)
+bool common_graph_run(Common * c, int steps, double omega, double xForce, const void * pdf, F record)
 {
-	if (!c->graphExec || c->graphSteps != steps || c->graphOmega != omega || c->graphForce != xForce) {
+	if (!c->graphExec || c->graphSteps != steps || c->graphOmega != omega || c->graphForce != xForce ||
+	    c->graphPdf != pdf) {
 		common_graph_drop(c);
 		(void)hipGetLastError();
 		if (!hip_ok(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture")) return false;
@@ -176,6 +181,7 @@ bool common_graph_run(Common * c, int steps, double omega, double xForce, F reco
 		c->graphSteps = steps;
 		c->graphOmega = omega;
 		c->graphForce = xForce;
+		c->graphPdf = pdf;
 	}
 	return hip_ok(hipGraphLaunch(c->graphExec, c->stream), "hipGraphLaunch");
 }

@@ -130,6 +130,8 @@ bool parse_kernel_args(const Parameters * p, KernelArgs * a, bool listKernel)
 	for (int i = 0; i < p->nKernelArgs; ++i) {
 		const char * s = p->KernelArgs[i];
 		auto is = [&](const char * x) { return !strcmp(s, x); };
+		for (const char * o : {"bs", "adj", "nt", "even-cap", "odd-order", "even-order", "odd-pairs", "vec"})
+			if (s[0] == '-' && !strcmp(s + (s[1] == '-' ? 2 : 1), o)) a->splitOption = 1;
 		if (is("-blk") || is("--blk")) {
 			int v;
 			if (!arg_int(p, i, &v, "-blk", 0, INT_MAX)) return false;
@@ -216,6 +218,13 @@ bool parse_kernel_args(const Parameters * p, KernelArgs * a, bool listKernel)
 			else return fail("argument -even-order requires down or up.");
 		} else if (is("-statistics") || is("--statistics")) {
 			a->statistics = 1;
+		} else if (is("-two-step") || is("--two-step")) {
+			if (i + 1 >= p->nKernelArgs) return fail("argument -two-step requires auto, on or off.");
+			const char * v = p->KernelArgs[++i];
+			if (!strcmp(v, "auto")) a->twoStep = -1;
+			else if (!strcmp(v, "on")) a->twoStep = 1;
+			else if (!strcmp(v, "off")) a->twoStep = 0;
+			else return fail("argument -two-step requires auto, on or off.");
 		} else if (is("-launch-events") || is("--launch-events")) {
 			if (i + 1 >= p->nKernelArgs) return fail("argument -launch-events requires on or off.");
 			const char * v = p->KernelArgs[++i];
@@ -249,7 +258,7 @@ bool parse_kernel_args(const Parameters * p, KernelArgs * a, bool listKernel)
 			if (listKernel) printf("  [-adj rle|full] [-shadow eager|lazy] [-odd-order band|group|plain] [-even-order down|up]\n");
 			else printf("  [-odd-pairs auto|on|off]\n");
 			printf("  [-force on|off] [-lambda <magic>] [-bs <threads per block>] [-nt on|off] [-even-cap on|off|force] [-quiet]\n");
-			printf("  [-launch-events on|off]\n");
+			printf("  [-launch-events on|off] [-two-step auto|on|off]\n");
 			return fail("kernel help requested.");
 		} else {
 			return fail("unknown kernel parameter: %s.", s);
