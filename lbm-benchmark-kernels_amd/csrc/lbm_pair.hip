@@ -166,26 +166,25 @@ __global__ __launch_bounds__(NT, WAVES) void k_pair(const typename Codec::S * __
 	};
 	for (int i = (int)threadIdx.x; i < 2 * E + 1; i += NT) ids[4 * P + i] = kNone;
 
-	S raw[19];                   // values of the next plane, in flight
+	S raw[19], raw1[19];         // values of the next plane (of plane x0), in flight
 	R ga[19], gb[19], old[5];    // even-step results of planes p and p - 1 in turn, c_x > 0 ones of p - 2
 	uint32_t offCur = offset_of(next_id(x0 - 1)), offPrev = kNone;
-	uint32_t idNext = next_id(x0);
+	uint32_t offNext = offset_of(next_id(x0)), idNext = next_id(x0 + 1);
 
-	auto load = [&](uint32_t off) __attribute__((always_inline)) {
+	auto load = [&](S (&to)[19], uint32_t off) __attribute__((always_inline)) {
 		Window w(src);
 #pragma unroll
 		for (int d = 0; d < 19; ++d) {
 			if (d) w.move(g.planeBytes);
-			get(raw[d], w.r, off);
+			get(to[d], w.r, off);
 		}
 	};
-	// Even step of plane p, and the values that leave a cell into LDS.
-	// FP16: as decoded values, which measured 2-3 % faster on dense lattices
-	// than 16-bit ones decoded when read.
-	auto even_part = [&](int p, R (&cur)[19], const R (&prev)[19]) __attribute__((always_inline)) {
+	// Even step of plane p.  FP16: the results as decoded values, which
+	// measured 2-3 % faster on dense lattices than 16-bit ones decoded when read.
+	auto even_part = [&](int p, R (&cur)[19], const S (&from)[19]) __attribute__((always_inline)) {
 #pragma unroll
 		for (int d = 0; d < 19; ++d) {
-			cur[d] = cod.dec(raw[d]);
+			cur[d] = cod.dec(from[d]);
 			if (EL) cur[d] = ft.add(cur[d], d);
 		}
 		trt_collide(cur, k);
@@ -194,6 +193,9 @@ __global__ __launch_bounds__(NT, WAVES) void k_pair(const typename Codec::S * __
 			for (int d = 0; d < 19; ++d) cur[d] = cod.dec(cod.enc(cur[d]));
 		}
 		ids[(p & 3) * P + t] = offCur;
+	};
+	// The values that leave a cell into LDS.
+	auto pass_on = [&](int p, const R (&cur)[19], const R (&prev)[19]) __attribute__((always_inline)) {
 		R * v = val + (p & 1) * 18 * P + t;
 #pragma unroll
 		for (int d = 0; d < 18; ++d)
@@ -247,7 +249,8 @@ __global__ __launch_bounds__(NT, WAVES) void k_pair(const typename Codec::S * __
 		w.move((uint32_t)(dC - at) * g.planeBytes);
 		put(cod.enc(f[dC]), w.r, own);
 	};
-	auto advance = [&](const R (&prev)[19], uint32_t offNext) __attribute__((always_inline)) {
+	// the c_x > 0 values of the plane before last, and the next plane
+	auto advance = [&](const R (&prev)[19]) __attribute__((always_inline)) {
 #pragma unroll
 		for (int d = 0; d < 18; ++d)
 			if (cx(d) > 0) old[cx(d) > 0 ? kAgeOf(d) : 0] = prev[d];
@@ -255,31 +258,28 @@ __global__ __launch_bounds__(NT, WAVES) void k_pair(const typename Codec::S * __
 		offCur = offNext;
 	};
 
-	// planes x0 - 1 and x0: even part only
-	load(offCur);
-#pragma unroll
-	for (int d = 0; d < 19; ++d) gb[d] = R(0);
-#pragma unroll
-	for (int j = 0; j < 5; ++j) old[j] = R(0);
-	auto lead = [&](int p, R (&cur)[19], const R (&prev)[19]) __attribute__((always_inline)) {
-		even_part(p, cur, prev);
-		const uint32_t offNext = offset_of(idNext);
-		load(offNext);
-		idNext = next_id(p + 2);
-		lds_barrier();
-		advance(prev, offNext);
-	};
+	// Planes x0 - 1 and x0: even part only, both loads in flight at once (with
+	// short segments the latency of one is a tenth of the launch).
+	load(raw, offCur);
+	load(raw1, offNext);
+	even_part(x0 - 1, ga, raw);
+	offPrev = offCur;
+	offCur = offNext;
+	offNext = offset_of(idNext);
+	load(raw, offNext);
+	idNext = next_id(x0 + 2);
+	even_part(x0, gb, raw1);
+	advance(ga);
 	auto step = [&](int p, R (&cur)[19], const R (&prev)[19]) __attribute__((always_inline)) {
-		even_part(p, cur, prev);
-		const uint32_t offNext = p < x1 ? offset_of(idNext) : kNone;
+		even_part(p, cur, raw);
+		pass_on(p, cur, prev);
+		offNext = p < x1 ? offset_of(idNext) : kNone;
 		lds_barrier();
-		load(offNext);
+		load(raw, offNext);
 		idNext = next_id(p + 2);
 		odd_part(p, prev);
-		advance(prev, offNext);
+		advance(prev);
 	};
-	lead(x0 - 1, ga, gb);
-	lead(x0, gb, ga);
 	// as many stores (of no cell) as a step issues: the loop's first wait for
 	// the loads may then count on them as all later ones do
 	{
@@ -304,15 +304,24 @@ constexpr int kShapes = 5;
 constexpr int kTileY[kShapes] = {13, 13, 5, 18, 28}, kTileZ[kShapes] = {32, 64, 32, 48, 32};
 constexpr int kTileThreads[kShapes] = {512, 1024, 256, 1024, 1024};
 
-// Per storage type and tile shape: the blocks that fit on a CU (registers,
-// LDS; 0: shape not used) and the time of one plane, base + perBlock * (blocks
-// running on a CU).  Fitted to lattices of 24^3 to 128^3; above the last-level
-// cache all times grow by about the same factor.
+// Estimated time of a launch, per storage type and tile shape, in a unit of
+// its own.  A block takes base + perBlock * (blocks on its CU) per plane, the
+// two halo planes of a segment together as many as `lead`; blocksPerCU fit on
+// a CU (registers, LDS; 0: shape not used).  Moving the values of a cell, the
+// tile's halo included, takes `cell`.  More blocks than fit run in rounds, of
+// which the last counts as full with the weight 1 - spread.  The constants
+// were chosen for the least average loss over 44 lattices of 24^3 to 256^3
+// (channels, pipes, blocks, porous media; up to 30 shapes and segment lengths
+// each): the plan takes on average 0.5 %, at most 5 %, longer than the best.
+// Per pair: aa-soa 64^3 FP32 17.3 -> 13.9 us against the smallest number of
+// planes in turn, porous 96^3 FP32 37.1 -> 33.0 us.
+struct TypeCost { double start, lead, cell, spread; };
 struct ShapeCost { int blocksPerCU; double base, perBlock; };
+constexpr TypeCost kTypeCost[3] = {{2.6, 1.1, 2.6e-5, 0.2}, {0.8, 1.0, 0.7e-5, 0.6}, {0.8, 0.7, 1.5e-5, 0.65}};
 constexpr ShapeCost kShapeCost[3][kShapes] = {
-	{{1, 2.5, 1.8}, {0, 0, 0}, {2, 1.7, 0.95}, {0, 0, 0}, {0, 0, 0}},
-	{{2, 1.5, 1.45}, {1, 2.6, 1.5}, {4, 1.1, 0.80}, {1, 2.7, 1.6}, {1, 2.8, 1.7}},
-	{{2, 1.6, 1.7}, {1, 3.0, 1.5}, {4, 1.2, 0.95}, {1, 3.1, 1.6}, {1, 3.2, 1.7}},
+	{{1, 2.66, 0}, {0, 0, 0}, {2, 1.1, 0.72}, {0, 0, 0}, {0, 0, 0}},
+	{{2, 0.63, 0.71}, {1, 1.8, 0}, {4, 0.62, 0.34}, {1, 2.05, 0}, {1, 2.1, 0}},
+	{{2, 0.67, 1.7}, {1, 3.5, 0}, {4, 0.7, 0.8}, {1, 3.5, 0}, {1, 3.95, 0}},
 };
 
 size_t pair_map_cells(const PairPlan & p) { return (size_t)(p.X + 2) * p.Y * p.Z; }
@@ -322,7 +331,7 @@ static bool face_fluid(const LatticeDesc * ld, int axis, int end)
 {
 	const int X = ld->Dims[0], Y = ld->Dims[1], Z = ld->Dims[2];
 	const int n[3] = {X, Y, Z};
-	const int u = (axis + 1) % 3, v = (axis + 2) % 3;
+	const int v = axis == 0 ? 1 : 0, u = 3 - axis - v;   // inner loop along x
 	for (int i = 0; i < n[u]; ++i)
 		for (int j = 0; j < n[v]; ++j) {
 			int c[3];
@@ -334,11 +343,12 @@ static bool face_fluid(const LatticeDesc * ld, int axis, int end)
 	return false;
 }
 
-// Tile shape and segment length with the least estimated time: the rounds of
-// blocks that the device runs, times the planes of a segment and the two of
-// its halo, times the time of one plane.
+// Tile shape and segment length with the least estimated time: that of the
+// blocks a CU runs one after the other or that of moving the values, whichever
+// is longer (with a smooth change between them).
 static void pair_shape(PairPlan * p, int nCU)
 {
+	const TypeCost & c = kTypeCost[p->prec];
 	double best = 0.0;
 	for (int s = 0; s < kShapes; ++s) {
 		const ShapeCost & w = kShapeCost[p->prec][s];
@@ -347,10 +357,14 @@ static void pair_shape(PairPlan * p, int nCU)
 		for (int n = 1; n <= p->X; ++n) {
 			const int seg = (p->X + n - 1) / n;
 			if ((p->X + seg - 1) / seg != n) continue;    // the same segments as a smaller n
-			const double r = (double)nTy * nTz * n / ((double)w.blocksPerCU * nCU);
-			const double rounds = r <= 1.0 ? 1.0 : 0.5 * (r + ceil(r));
-			const double running = w.blocksPerCU * (r < 1.0 ? r : 1.0);
-			const double t = rounds * (seg + 2) * (w.base + w.perBlock * running);
+			const double blocks = (double)nTy * nTz * n, r = blocks / ((double)w.blocksPerCU * nCU);
+			const double rounds = r <= 1.0 ? 1.0 : c.spread * r + (1.0 - c.spread) * ceil(r);
+			const double idle = r <= 1.0 ? 1.0 : rounds / r;
+			const double onCU = fmin(w.blocksPerCU, ceil(blocks / nCU));
+			const double planes = seg + c.lead;
+			const double inTurn = rounds * planes * (w.base + w.perBlock * onCU);
+			const double moved = blocks * planes * (kTileY[s] + 1) * (kTileZ[s] + 1) * c.cell * idle * idle;
+			const double t = c.start + cbrt(inTurn * inTurn * inTurn + moved * moved * moved);
 			if (best == 0.0 || t < best) {
 				best = t;
 				p->shape = s;
