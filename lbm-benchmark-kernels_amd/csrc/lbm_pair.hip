@@ -315,9 +315,13 @@ constexpr int kTileThreads[kShapes] = {512, 1024, 256, 1024, 1024};
 // each): the plan takes on average 0.5 %, at most 5 %, longer than the best.
 // Per pair: aa-soa 64^3 FP32 17.3 -> 13.9 us against the smallest number of
 // planes in turn, porous 96^3 FP32 37.1 -> 33.0 us.
-struct TypeCost { double start, lead, cell, spread; };
+// The list kernel's even and odd launch cost splitLaunch + splitNode * nodes in
+// the same unit: they skip solid cells, a tile's lanes do not.
+struct TypeCost { double start, lead, cell, spread, splitLaunch, splitNode; };
 struct ShapeCost { int blocksPerCU; double base, perBlock; };
-constexpr TypeCost kTypeCost[3] = {{2.6, 1.1, 2.6e-5, 0.2}, {0.8, 1.0, 0.7e-5, 0.6}, {0.8, 0.7, 1.5e-5, 0.65}};
+constexpr TypeCost kTypeCost[3] = {{2.6, 1.1, 2.6e-5, 0.2, 10.0, 7.5e-5},
+                                     {0.8, 1.0, 0.7e-5, 0.6, 4.0, 2.1e-5},
+                                     {0.8, 0.7, 1.5e-5, 0.65, 5.2, 2.3e-5}};
 constexpr ShapeCost kShapeCost[3][kShapes] = {
 	{{1, 2.66, 0}, {0, 0, 0}, {2, 1.1, 0.72}, {0, 0, 0}, {0, 0, 0}},
 	{{2, 0.63, 0.71}, {1, 1.8, 0}, {4, 0.62, 0.34}, {1, 2.05, 0}, {1, 2.1, 0}},
@@ -345,8 +349,8 @@ static bool face_fluid(const LatticeDesc * ld, int axis, int end)
 
 // Tile shape and segment length with the least estimated time: that of the
 // blocks a CU runs one after the other or that of moving the values, whichever
-// is longer (with a smooth change between them).
-static void pair_shape(PairPlan * p, int nCU)
+// is longer (with a smooth change between them).  Returns that time.
+static double pair_shape(PairPlan * p, int nCU)
 {
 	const TypeCost & c = kTypeCost[p->prec];
 	double best = 0.0;
@@ -375,6 +379,7 @@ static void pair_shape(PairPlan * p, int nCU)
 			}
 		}
 	}
+	return best;
 }
 
 void pair_plan(PairPlan * p, const KernelArgs & a, int nCU, const LatticeDesc * ld, uint64_t plane, bool openFaces)
@@ -416,15 +421,22 @@ void pair_plan(PairPlan * p, const KernelArgs & a, int nCU, const LatticeDesc * 
 	p->z0 = fluid[2][0] ? 0 : 1;
 	p->z1 = p->Z - (fluid[2][1] ? 0 : 1);
 	if (p->y1 <= p->y0 || p->z1 <= p->z0) return;
-	// The list kernel's launches skip solid cells, a tile's lanes do not.
-	// Speed-up over the two launches at fluid fractions 0.55 / 0.65 / 0.8 / 1:
-	// FP64 0.96 / 1.08 / 1.05-1.4 / 1.2-1.4, FP32 0.93-1.08 / 0.99-1.08 /
-	// 1.05-1.5 / 1.2-1.5, FP16 0.7-1.06 at 0.8 and 1.02-1.2 at 1.  The full-array
-	// launches visit every cell: 1.04-2.1 in all types, also at 0.55.
-	const double least = p->useDense ? 0.0 : p->prec == PREC_FP64 ? 0.6 : p->prec == PREC_FP32S ? 0.65 : 0.9;
-	const double cells = (double)p->X * (p->y1 - p->y0) * (p->z1 - p->z0);
-	if (a.twoStep < 0 && (double)ld->nFluid < least * cells) return;
-	pair_shape(p, nCU > 0 ? nCU : 256);
+	// Speed-up over the list kernel's two launches, porous media and channels:
+	// FP64 1.14-1.43 below 64^3 and 1.05-1.3 above at a fluid fraction of 0.65
+	// and more, 0.79-1.15 below that; FP32 1.2-1.58, 1.0-1.3 and 0.91-1.01; FP16
+	// 1.04-1.68 below 64^3, above it 0.71-1.07 and only for dense lattices that
+	// the tiles cover well 1.05 (128^3) to 1.21 (256^3).  The comparison below
+	// takes most that gain more than 5 % and, of 130 lattices, two that lose
+	// 5-13 % (FP32 109x167x147 at 0.85; FP64 176x134x188 at 0.53).  aa-soa's launches visit every cell: 1.04-2.3 in all
+	// types, also at 0.55.
+	// Where one array fits into the 256 MiB last-level cache and two hardly do, the
+	// launch reads more from memory than the separate ones do: FP64 121x87x131
+	// at 0.7 and 98x130x105 at 0.57 0.86-0.90, FP32 160^3 at 0.55 0.91.
+	double t = pair_shape(p, nCU > 0 ? nCU : 256);
+	const TypeCost & c = kTypeCost[p->prec];
+	const double bytes = 19.0 * (double)elem * ld->nFluid, cache = 256.0 * (1 << 20);
+	if (bytes < cache && 2 * bytes > 0.8 * cache) t *= 1.2;
+	if (a.twoStep < 0 && !p->useDense && t > c.splitLaunch + c.splitNode * ld->nFluid) return;
 	p->use = true;
 }
 
