@@ -10,27 +10,30 @@ A "step" is one LBM timestep over all fluid nodes.  The lattice, list and
 adjacency are built on and resident in HBM before timing; the timed region
 is exactly --steps timesteps (rounded up to even: AA steps come in
 even/odd pairs), measured with HIP events recorded on the kernel's stream
-around the step loop and around every launch.  value = nFluid * steps /
-time / 1e6 (src/Main.c:594).
+around the step loop.  value = nFluid * steps / time / 1e6
+(src/Main.c:594).
 
 --prec fp32s / fp16s run the shifted-storage variants (deviations f - w in
 FP32 or scaled binary16, collision in FP32) on the same workload: 4 or 2 B
 per value instead of 8; the default and headline is FP64.
 
-roofline: the odd-step kernel (the longer of the two).  Algorithmic bytes
-per fluid node: the list-AA odd-step balance, 19 loads + 19 stores of 8 B
-plus 18 int32 adjacency entries = 376 B (doc/main.rst:347), the adjacency
-compression not credited; even step 304 B (the two average 340 B/FLUP).
-achieved = 376 B * nFluid / mean odd-launch time.  The bytes the kernel
-needs with the run-compressed adjacency (304 B plus 72 B per run and 12 B
-per 64-node wavefront, reported by the library: 317.8 B here) give the
-"moved" figures beside it.  traffic: HBM bytes per odd launch from rocprofv3
-FETCH_SIZE + WRITE_SIZE scaled by a copy kernel of known size
-(profiles/list_odd_porous256_traffic.json), null if absent; hbm_pair: the
-measured bytes of an even + odd pair from the same file over this run's
-even + odd launch time (the achieved HBM rate of a step pair).  The copy and
-update-19 bandwidths of the device are measured in the same run as
-yardsticks (the reference rates its kernels against update-19 bandwidth).
+roofline: the launch of the timed steps.  By default that is k_pair, an even
+and an odd step in one launch: its bytes are the 19 loads and 19 stores of a
+fluid node (304 B) and the 4 B of the index map, once per two steps; achieved
+= 308 B * nFluid / (time of two steps).  traffic: HBM bytes per launch from
+rocprofv3 FETCH_SIZE + WRITE_SIZE scaled by a copy kernel of known size
+(profiles/list_pair_porous256_traffic.json), null if absent.  The even and odd
+launches, which a run with per-launch events uses, are measured in a second
+run of at most 100 steps and stand in separate_launches: bytes per fluid node
+are the list-AA balance, 19 loads + 19 stores of 8 B plus, in the odd step, 18
+int32 adjacency entries = 376 B (doc/main.rst:347), the adjacency compression
+not credited; "moved" counts the bytes the odd kernel needs with the
+run-compressed adjacency (304 B plus 72 B per run and 12 B per 64-node
+wavefront, reported by the library: 317.8 B here).  Where the library does not
+launch pairs (-two-step off, FP16 here) the odd launch is the roofline's kernel.
+step_average_gbs rates the timed steps on the list-AA balance.  The copy and
+update-19 bandwidths of the device are measured in the same run as yardsticks
+(the reference rates its kernels against update-19 bandwidth).
 
 cpu_baseline: the reference's own list-aa-pv-soa (benchmark build, compiled
 from its sources into oracle/_ref) on the same geometry, OpenMP on the host
@@ -49,10 +52,12 @@ plain path queued in arrival order.
 from __future__ import annotations
 
 import argparse
+import ctypes as C
 import json
 import os
 import subprocess
 import sys
+import tempfile
 import time
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
@@ -62,7 +67,27 @@ GEOMETRY = "porous-6-0.8-42"
 DIMS = (256, 256, 256)
 OMEGA, LAMBDA, XFORCE = 1.2, 0.1875, 1e-6
 PEAK_GBS = 8000.0
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "list_odd_porous256_traffic.json")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "list_pair_porous256_traffic.json")
+TRAFFIC_FILE_ODD = os.path.join(ROOT, "profiles", "list_odd_porous256_traffic.json")
+
+
+def build_report(build):
+    """(result of build(), what the library printed on stdout meanwhile,
+    passed on to stderr)."""
+    with tempfile.TemporaryFile() as tmp:
+        sys.stdout.flush()
+        keep = os.dup(1)
+        os.dup2(tmp.fileno(), 1)
+        try:
+            result = build()
+        finally:
+            C.CDLL(None).fflush(None)
+            os.dup2(keep, 1)
+            os.close(keep)
+        tmp.seek(0)
+        text = tmp.read().decode()
+    print(text, end="", file=sys.stderr, flush=True)
+    return result, text
 
 
 def cpu_baseline(mask, dims, periodic, n_fluid, steps):
@@ -477,7 +502,7 @@ def aa_mode(args, lbm):
     (the small configuration the reference also runs on its CPU) and 256^3,
     the latter also with shifted FP32 / FP16 storage.  Throughput from a run
     without per-launch events, even/odd launch averages from a second run
-    with them."""
+    with them (which launches the two steps one by one)."""
     out = {}
     for edge, steps, prec in ((64, 1000, "fp64"), (256, 200, "fp64"), (256, 200, "fp32s"), (256, 200, "fp16s")):
         geo = lbm.Geometry.from_string("channel", (edge, edge, edge), (1, 0, 0))
@@ -563,12 +588,13 @@ def main():
     geo = lbm.Geometry.from_string(GEOMETRY, DIMS)
     nf = geo.n_fluid
     print(f"bench: {GEOMETRY} {DIMS} nFluid={nf} steps={steps} warmup={warm}", file=sys.stderr, flush=True)
-    k = lbm.Kernel("list-aa-pv-soa", geo, ["-lambda", repr(LAMBDA), "-prec", args.prec] + args.kernel_args.split())
+    k, report = build_report(lambda: lbm.Kernel("list-aa-pv-soa", geo, ["-lambda", repr(LAMBDA), "-prec", args.prec] +
+                                                args.kernel_args.split()))
+    pairs = "two-step launch" in report
     info = k.list_info()
     b_even = info.bytesPerFlupEven
     k.set_initial_weights()
     k.set_shadow_download(False)
-    k.set_launch_events(True)       # even/odd launch averages for the roofline, over the timed steps
     cd = lbm.case_data(omega=OMEGA, xforce=XFORCE, iterations=warm)
     if warm:
         k.run(cd)
@@ -579,13 +605,19 @@ def main():
     t = k.timings()
     loop_s = t.loopMs / 1e3
     value = nf * steps / loop_s / 1e6
+    k.set_launch_events(True)       # even/odd launch averages
+    cd.MaxIterations = min(steps, 100)
+    k.run(cd)
+    te = k.timings()
     b_moved = info.bytesPerFlupOdd              # with the run-compressed adjacency
     b_odd = b_even + 18 * 4                     # list-AA odd balance: full int32 adjacency
-    odd_gbs = b_odd * nf / (t.oddMsAvg / 1e3) / 1e9
-    moved_gbs = b_moved * nf / (t.oddMsAvg / 1e3) / 1e9
-    even_gbs = b_even * nf / (t.evenMsAvg / 1e3) / 1e9
-    print(f"bench: {value:.1f} MFLUP/s loop {t.loopMs:.2f} ms wall {wall * 1e3:.2f} ms even {t.evenMsAvg:.4f} ms "
-          f"({even_gbs:.0f} GB/s) odd {t.oddMsAvg:.4f} ms ({odd_gbs:.0f} GB/s at {b_odd} B, {moved_gbs:.0f} GB/s "
+    odd_gbs = b_odd * nf / (te.oddMsAvg / 1e3) / 1e9
+    moved_gbs = b_moved * nf / (te.oddMsAvg / 1e3) / 1e9
+    b_pair = b_even + 4                         # PDFs in and out, index map
+    pair_gbs = b_pair * nf / (2 * loop_s / steps) / 1e9
+    even_gbs = b_even * nf / (te.evenMsAvg / 1e3) / 1e9
+    print(f"bench: {value:.1f} MFLUP/s loop {t.loopMs:.2f} ms wall {wall * 1e3:.2f} ms even {te.evenMsAvg:.4f} ms "
+          f"({even_gbs:.0f} GB/s) odd {te.oddMsAvg:.4f} ms ({odd_gbs:.0f} GB/s at {b_odd} B, {moved_gbs:.0f} GB/s "
           f"at {b_moved:.1f} B) runs={info.nRuns}", file=sys.stderr, flush=True)
     mask = geo.mask.reshape(-1).copy()
     periodic = geo.periodic
@@ -595,16 +627,16 @@ def main():
     print(f"bench: yardsticks copy {yard['copy_gbs']:.0f} GB/s update-19 {yard['update19_gbs']:.0f} GB/s",
           file=sys.stderr, flush=True)
 
-    traffic, pair = None, None
-    if args.prec == "fp64" and os.path.exists(TRAFFIC_FILE):
-        with open(TRAFFIC_FILE) as f:
-            tf = json.load(f)
-        traffic = tf.get("bytes_per_launch")
-        if "even" in tf and "odd" in tf:
-            # measured HBM bytes of an even + odd pair over this run's pair time
-            pb = tf["even"]["bytes_per_launch"] + tf["odd"]["bytes_per_launch"]
-            pair_gbs = pb / ((t.evenMsAvg + t.oddMsAvg) / 1e3) / 1e9
-            pair = {"bytes": pb, "achieved_gbs": round(pair_gbs, 1), "frac": round(pair_gbs / PEAK_GBS, 4)}
+    traffic, hbm = None, None
+    traffic_file = TRAFFIC_FILE if pairs else TRAFFIC_FILE_ODD
+    if args.prec == "fp64" and os.path.exists(traffic_file):
+        with open(traffic_file) as f:
+            traffic = json.load(f).get("bytes_per_launch")
+    if traffic is not None:
+        # measured HBM bytes of the launch over this run's time of it
+        hbm_gbs = traffic / ((2 * loop_s / steps) if pairs else te.oddMsAvg / 1e3) / 1e9
+        hbm = {"bytes": traffic, "achieved_gbs": round(hbm_gbs, 1), "frac": round(hbm_gbs / PEAK_GBS, 4),
+               "frac_of_update19": round(hbm_gbs / yard["update19_gbs"], 4)}
 
     base = None
     if not args.no_cpu_baseline:
@@ -636,24 +668,31 @@ def main():
         "config": {"workload": "list-aa-pv-soa, 256x256x256 porous medium (spheres r=6, porosity<=0.80, seed 42), "
                                f"x periodic, omega 1.2, Lambda 3/16, Luo force 1e-6, {label}",
                    "n_fluid": nf, "n_cells_padded": info.nCells, "device": dev.get("name")},
-        "roofline": {"bound": "hbm", "kernel": "k_list_odd (odd AA step, run-compressed adjacency)",
-                     "scope": "frac is the dominant kernel's (the odd step); step_average_frac is the whole step's",
-                     "achieved": round(odd_gbs, 1), "peak": PEAK_GBS, "unit": "GB/s",
-                     "frac": round(odd_gbs / PEAK_GBS, 4), "traffic": traffic,
-                     "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT) if traffic is not None else None,
-                     "hbm_pair": pair,
-                     "bytes_per_flup": b_odd,
-                     "bytes_basis": "list-AA odd balance: 19 loads + 19 stores + 18 int32 adjacency entries per "
+        "roofline": {"bound": "hbm",
+                     "kernel": "k_pair (an even and an odd AA step in one launch)" if pairs else
+                               "k_list_odd (odd AA step, run-compressed adjacency)",
+                     "scope": "frac is the named kernel's; step_average_frac is the whole step's on the list-AA balance",
+                     "achieved": round(pair_gbs if pairs else odd_gbs, 1), "peak": PEAK_GBS, "unit": "GB/s",
+                     "frac": round((pair_gbs if pairs else odd_gbs) / PEAK_GBS, 4), "traffic": traffic,
+                     "traffic_source": os.path.relpath(traffic_file, ROOT) if traffic is not None else None,
+                     "hbm": hbm,
+                     "bytes_per_flup": b_pair / 2 if pairs else b_odd,
+                     "bytes_basis": "19 loads + 19 stores + 4 B of the index map per node and two steps" if pairs else
+                                    "list-AA odd balance: 19 loads + 19 stores + 18 int32 adjacency entries per "
                                     "node, adjacency compression not credited",
-                     "moved": {"bytes_per_flup": round(b_moved, 3), "achieved": round(moved_gbs, 1),
-                               "frac": round(moved_gbs / PEAK_GBS, 4)},
-                     "odd_ms_avg": t.oddMsAvg, "runs_per_wave_cut": runs_wave,
-                     "even_kernel": {"achieved": round(even_gbs, 1), "frac": round(even_gbs / PEAK_GBS, 4),
-                                     "bytes_per_flup": b_even, "ms_avg": t.evenMsAvg},
+                     "ms_avg": 2 * t.loopMs / steps if pairs else te.oddMsAvg,
                      "step_average_gbs": round((b_even + b_odd) / 2 * nf * steps / loop_s / 1e9, 1),
-                     "yardsticks_gbs": {"copy": round(yard["copy_gbs"], 1), "update19": round(yard["update19_gbs"], 1)},
-                     "moved_frac_of_copy": round(moved_gbs / yard["copy_gbs"], 4),
-                     "step_average_frac": round((b_even + b_odd) / 2 * nf * steps / loop_s / 1e9 / PEAK_GBS, 4)},
+                     "step_average_frac": round((b_even + b_odd) / 2 * nf * steps / loop_s / 1e9 / PEAK_GBS, 4),
+                     "yardsticks_gbs": {"copy": round(yard["copy_gbs"], 1), "update19": round(yard["update19_gbs"], 1)}},
+        "separate_launches": {"odd_ms_avg": te.oddMsAvg, "even_ms_avg": te.evenMsAvg,
+                              "mflups": round(nf * cd.MaxIterations / (te.loopMs / 1e3) / 1e6, 2),
+                              "odd": {"bytes_per_flup": b_odd, "achieved_gbs": round(odd_gbs, 1),
+                                      "frac": round(odd_gbs / PEAK_GBS, 4), "runs_per_wave_cut": runs_wave,
+                                      "moved": {"bytes_per_flup": round(b_moved, 3), "achieved_gbs": round(moved_gbs, 1),
+                                                "frac": round(moved_gbs / PEAK_GBS, 4),
+                                                "frac_of_copy": round(moved_gbs / yard["copy_gbs"], 4)}},
+                              "even": {"bytes_per_flup": b_even, "achieved_gbs": round(even_gbs, 1),
+                                       "frac": round(even_gbs / PEAK_GBS, 4)}},
         "cpu_baseline": base,
         "solves": solves,
         "serving": serving,

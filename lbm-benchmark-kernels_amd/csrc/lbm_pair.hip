@@ -427,8 +427,8 @@ void pair_plan(PairPlan * p, const KernelArgs & a, int nCU, const LatticeDesc * 
 	// 1.04-1.68 below 64^3, above it 0.71-1.07 and only for dense lattices that
 	// the tiles cover well 1.05 (128^3) to 1.21 (256^3).  The comparison below
 	// takes most that gain more than 5 % and, of 130 lattices, two that lose
-	// 5-13 % (FP32 109x167x147 at 0.85; FP64 176x134x188 at 0.53).  aa-soa's launches visit every cell: 1.04-2.3 in all
-	// types, also at 0.55.
+	// 5-13 % (FP32 109x167x147 at 0.85; FP64 176x134x188 at 0.53).  aa-soa's
+	// launches visit every cell: 1.04-2.5 in all types, also at 0.55.
 	// Where one array fits into the 256 MiB last-level cache and two hardly do, the
 	// launch reads more from memory than the separate ones do: FP64 121x87x131
 	// at 0.7 and 98x130x105 at 0.57 0.86-0.90, FP32 160^3 at 0.55 0.91.
