@@ -426,16 +426,18 @@ void pair_plan(PairPlan * p, const KernelArgs & a, int nCU, const LatticeDesc * 
 	// and more, 0.79-1.15 below that; FP32 1.2-1.58, 1.0-1.3 and 0.91-1.01; FP16
 	// 1.04-1.68 below 64^3, above it 0.71-1.07 and only for dense lattices that
 	// the tiles cover well 1.05 (128^3) to 1.21 (256^3).  The comparison below
-	// takes most that gain more than 5 % and, of 130 lattices, two that lose
-	// 5-13 % (FP32 109x167x147 at 0.85; FP64 176x134x188 at 0.53).  aa-soa's
-	// launches visit every cell: 1.04-2.5 in all types, also at 0.55.
-	// Where one array fits into the 256 MiB last-level cache and two hardly do, the
-	// launch reads more from memory than the separate ones do: FP64 121x87x131
-	// at 0.7 and 98x130x105 at 0.57 0.86-0.90, FP32 160^3 at 0.55 0.91.
+	// takes most that gain more than 5 % and, of 160 lattices, one that loses
+	// more than 3 % (FP64 176x134x188 at 0.53, 0.96).  aa-soa's launches visit
+	// every cell: 1.04-2.5 in all types, also at 0.55.
+	// Where the separate launches' array fits well into the 256 MiB last-level
+	// cache and two arrays hardly do, the launch reads more from memory than they
+	// do.  At 102 to 187 MiB: FP32 0.81-1.0 and FP64 0.86-1.05 where the
+	// estimates are within a factor of 1.45, 1.0-1.15 where they are further
+	// apart; 1.03-1.29 in both types from 188 MiB on.
 	double t = pair_shape(p, nCU > 0 ? nCU : 256);
 	const TypeCost & c = kTypeCost[p->prec];
 	const double bytes = 19.0 * (double)elem * ld->nFluid, cache = 256.0 * (1 << 20);
-	if (bytes < cache && 2 * bytes > 0.8 * cache) t *= 1.2;
+	if (bytes > 0.4 * cache && bytes < 0.73 * cache) t *= 1.45;
 	if (a.twoStep < 0 && !p->useDense && t > c.splitLaunch + c.splitNode * ld->nFluid) return;
 	p->use = true;
 }
