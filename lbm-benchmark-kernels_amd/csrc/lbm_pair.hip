@@ -25,9 +25,18 @@
 // registers until then, so that LDS keeps 18 values per cell and parity; two
 // parities make one barrier per plane enough.
 //
-// What bounds it (256^3, MI355X): per lane and direction one load and one
-// store, at about 9.5 bytes per clock and CU over all CUs -- the rate of a
-// plain copy.
+// What bounds it (MI355X), and the two launches' time -> this one's per pair:
+// * large lattices: HBM.  256^3 list FP64 moves 4.67 GB (13 % over the PDFs
+//   once in and out: halos, lines shared with solid cells) at 4.07 TB/s, 1.50
+//   -> 1.15 ms; aa-soa FP64 5.62 GB at 4.5 TB/s, 1.81 -> 1.24 ms, FP32 2.76 GB
+//   at 4.45 TB/s, 0.94 -> 0.62 ms; 19 streams updated in place reach 4.7 TB/s.
+// * FP16, and FP32 up to about 100^3: vector issue, 566 and 484 instructions
+//   per lane and plane (470 and 394 of them arithmetic) at four wavefronts per
+//   SIMD: pipe 129x83x110 FP16 52.2 -> 39.4 us.
+// * FP64 up to about 100^3: loads of the halos and the lead planes, 1.8 to 2
+//   times the cells' own with segments of a few planes: 64^3 29.6 -> 21.4 us.
+// * 24^3 to 40^3: the latency of map, PDFs and stores in turn: 6 to 8 us
+//   against 8 to 14 us.
 #include "lbm_pair.h"
 
 #include <math.h>
@@ -299,7 +308,11 @@ __global__ __launch_bounds__(NT, WAVES) void k_pair(const typename Codec::S * __
 // ------------------------------------------------------------ launch shapes
 // Tile shapes (cells in y and z, threads).  A block holds its tile's state in
 // registers and LDS: at most 512 cells with halo in FP64, 1024 in the narrow
-// types.
+// types.  Rows of 32 cells and more keep whole lines in a row's accesses;
+// 256^3 FP64 1.20 ms with 13 x 32, 1.33 with 10 x 40, 1.27 with 8 x 48, 1.35
+// with 17 x 24.  The other shapes fit ragged planes (18 x 48, 28 x 32: pipe
+// 129x83x110 FP16 39.5 against 40.7 us and more), small ones (5 x 32: 24^3 7.0
+// against 9.2 us) and large narrow ones (13 x 64).
 constexpr int kShapes = 5;
 constexpr int kTileY[kShapes] = {13, 13, 5, 18, 28}, kTileZ[kShapes] = {32, 64, 32, 48, 32};
 constexpr int kTileThreads[kShapes] = {512, 1024, 256, 1024, 1024};
