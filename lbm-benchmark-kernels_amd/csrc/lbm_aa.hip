@@ -724,18 +724,20 @@ static void aa_dense_copy(AaData * A, bool toDense)
 }
 
 // The arrays of the two-step launch; the number of fluid cells in the mask to
-// *count (device).
-static void aa_build_pair(AaData * A, const LatticeDesc * ld, uint32_t * count, hipStream_t s)
+// *count (device).  Launches before this call are checked by the caller:
+// pair_alloc leaves no error behind where it takes no memory.
+static bool aa_build_pair(AaData * A, const LatticeDesc * ld, uint32_t * count, hipStream_t s)
 {
 	const AaGeom & g = A->g;
 	PairPlan & p = A->pair;
 	pair_plan(&p, A->c.args, A->c.nCU, ld, 0, false);
 	pair_alloc(&p);
-	if (!p.use) return;
+	if (!p.use) return true;
 	const uint32_t rows = (uint32_t)g.X * g.Y;
 	k_aa_row_counts<<<(rows + 255) / 256, 256, 0, s>>>(A->dFluid, g, p.rows);
 	scan_exclusive(p.rows, rows, count, s);
 	k_aa_pair_map<<<(unsigned)((pair_map_cells(p) + 255) / 256), 256, 0, s>>>(A->dFluid, g, p.rows, p.map);
+	return hip_ok(hipGetLastError(), "cell map kernel");
 }
 
 // Host copy of the current state for the output functions' GetNode.
@@ -1110,8 +1112,8 @@ void D3Q19AaInit_AaSoAHip(LatticeDesc * ld, KernelData ** kernelData, Parameters
 		(void)hipGetLastError();
 		k_aa_info<<<(unsigned)((nTotal + 255) / 256), 256, 0, s>>>(dMask, g, A->dInfo, dCount);
 		k_aa_fluid_bits<<<(unsigned)((nWords + 255) / 256), 256, 0, s>>>(A->dInfo, g, A->dFluid);
-		aa_build_pair(A, ld, dCount + 1, s);
 		if (!hip_ok(hipGetLastError(), "cell info kernel")) break;
+		if (!aa_build_pair(A, ld, dCount + 1, s)) break;
 		if (!hip_ok(hipMemcpyAsync(hCount, dCount, sizeof(hCount), hipMemcpyDeviceToHost, s), "count download")) break;
 		A->hPdf = host_alloc(aa_bytes(A));
 		if (!A->hPdf) { fail("allocating host lattice failed: %zu bytes.", aa_bytes(A)); break; }

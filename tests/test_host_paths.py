@@ -1,0 +1,83 @@
+"""The host side of liblbmhip.so without a device: which launches a call
+makes, what it allocates and what it does when an allocation or a launch
+fails.  Each test runs a script in a child process whose HIP runtime is the
+stub of tests/stub_hip (device memory out of a budget, launches logged)."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import PKG, ROOT
+
+STUB = os.path.join(ROOT, "tests", "stub_hip", "hip_stub.c")
+pytestmark = pytest.mark.skipif(shutil.which("gcc") is None or not os.path.exists("/opt/rocm/include/hip"),
+                                reason="needs gcc and the HIP headers")
+
+PRELUDE = """
+import ctypes as C, sys
+sys.path.insert(0, {pkg!r})
+import lbm_amd as lbm
+S = C.CDLL({stub!r})
+S.stub_log.restype = C.c_char_p
+
+def free_bytes(n=None):
+    v = C.c_size_t.in_dll(S, "stub_free")
+    if n is not None:
+        v.value = n
+    return v.value
+
+def fail_launch(name):
+    C.memmove(C.addressof(C.c_char.in_dll(S, "stub_fail_launch")), name.encode() + bytes(1), len(name) + 1)
+
+def fail_call(name):
+    C.memmove(C.addressof(C.c_char.in_dll(S, "stub_fail_call")), name.encode() + bytes(1), len(name) + 1)
+
+def log():
+    # lines since the last call
+    text = S.stub_log().decode().splitlines()
+    S.stub_clear()
+    return text
+
+def launches(name):
+    return sum(line.startswith("launch") and name in line for line in log())
+
+def kernel(name, dims, args=(), periodic=(1, 0, 0), geo="channel"):
+    g = lbm.Geometry.from_string(geo, dims, periodic)
+    C.c_uint32.in_dll(S, "stub_count").value = g.n_fluid
+    return lbm.Kernel(name, g, ["-quiet"] + list(args))
+
+def case(steps, **kw):
+    return lbm.case_data(iterations=steps, **kw)
+"""
+
+
+@pytest.fixture(scope="session")
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", STUB, "-o", out,
+                    "-lpthread"], check=True, capture_output=True)
+
+    def run(script):
+        env = dict(os.environ, LD_PRELOAD=out)
+        r = subprocess.run([sys.executable, "-c", PRELUDE.format(pkg=PKG, stub=out) + textwrap.dedent(script)],
+                           capture_output=True, text=True, env=env, timeout=120)
+        assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-3000:])
+    return run
+
+
+def test_init_reports_a_failed_launch_when_memory_is_short(stub):
+    """aa-soa's Init reports a launch that failed also where the arrays of the
+    two-step launch do not fit."""
+    stub("""
+        free_bytes(8 << 20)
+        fail_launch("k_aa_info")
+        try:
+            kernel("aa-soa", (40, 24, 24))
+        except RuntimeError as e:
+            assert "cell info kernel" in str(e), e
+        else:
+            raise AssertionError("Init succeeded")
+    """)
