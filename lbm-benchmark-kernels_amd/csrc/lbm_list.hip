@@ -469,8 +469,11 @@ static bool list_build_pair(ListData * L)
 	(void)hipGetLastError();
 	k_list_pair_map<<<(unsigned)((pair_map_cells(L->pair) + 255) / 256), 256, 0, L->c.stream>>>(
 		L->dGrid, L->dims[0], L->dims[1], L->dims[2], L->periodic[0], L->pair.map);
-	return hip_ok(hipGetLastError(), "cell map kernel") &&
-	       hip_ok(hipMemsetAsync(L->pair.other, 0, elem_bytes(L->c.args.prec) * 19 * (size_t)L->nCells, L->c.stream), "hipMemset");
+	if (hip_ok(hipGetLastError(), "cell map kernel") &&
+	    hip_ok(hipMemsetAsync(L->pair.other, 0, elem_bytes(L->c.args.prec) * 19 * (size_t)L->nCells, L->c.stream), "hipMemset"))
+		return true;
+	pair_release(&L->pair);      // a later call must not find a map that was never written
+	return false;
 }
 
 // ------------------------------------------------------------- Kernel()

@@ -46,6 +46,9 @@ size_t pair_map_cells(const PairPlan & p);
 // take more than half of the device's free memory the lattice is left to the
 // separate kernels.
 void pair_alloc(PairPlan * p);
+// Frees the arrays; the plan stays, and the next pair_alloc takes them again.
+void pair_release(PairPlan * p);
+// The same, and the lattice is stepped by the separate kernels from now on.
 void pair_free(PairPlan * p);
 
 // The launch shape, as a line of Init's report.

@@ -489,10 +489,16 @@ void pair_alloc(PairPlan * p)
 	p->map = (uint32_t *)at;
 }
 
-void pair_free(PairPlan * p)
+void pair_release(PairPlan * p)
 {
 	(void)hipFree(p->block);
 	p->block = nullptr;
+	p->current = false;
+}
+
+void pair_free(PairPlan * p)
+{
+	pair_release(p);
 	p->use = false;
 }
 

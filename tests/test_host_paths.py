@@ -81,3 +81,26 @@ def test_init_reports_a_failed_launch_when_memory_is_short(stub):
         else:
             raise AssertionError("Init succeeded")
     """)
+
+
+@pytest.mark.parametrize("what", ["launch", "memset"])
+def test_list_arrays_are_built_again_after_a_failure(stub, what):
+    """A Kernel() call that could not fill the cell map or clear the second
+    array fails, and the next call builds both before it uses them."""
+    stub(f"""
+        k = kernel("list-aa-pv-soa", (20, 20, 20), ["-two-step", "on"])
+        what = {what!r}
+        fail_launch("k_list_pair_map") if what == "launch" else fail_call("memset")
+        try:
+            k.run(case(4))
+        except RuntimeError as e:
+            assert ("cell map kernel" if what == "launch" else "hipMemset") in str(e), e
+        else:
+            raise AssertionError("no error")
+        fail_launch("")
+        fail_call("")
+        log()
+        k.run(case(4))
+        lines = [line for line in log() if line.startswith("launch")]
+        assert "k_list_pair_map" in lines[0] and all("k_pair" in line for line in lines[1:]), lines
+    """)
