@@ -730,7 +730,7 @@ static bool aa_build_pair(AaData * A, const LatticeDesc * ld, uint32_t * count, 
 {
 	const AaGeom & g = A->g;
 	PairPlan & p = A->pair;
-	pair_plan(&p, A->c.args, A->c.nCU, ld, 0, false);
+	pair_plan(&p, A->c, ld, 0, false);
 	pair_alloc(&p);
 	if (!p.use) return true;
 	const uint32_t rows = (uint32_t)g.X * g.Y;

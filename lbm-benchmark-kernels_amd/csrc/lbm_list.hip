@@ -1053,7 +1053,7 @@ void D3Q19ListAaPvInit_PushSoAHip(LatticeDesc * ld, KernelData ** kernelData, Pa
 	if (!dev_alloc((void **)&L->dPdfOwn, pdfBytes, "device lattice")) { list_release(L); return; }
 	L->dPdf = L->dPdfOwn;
 	if (!hip_ok(hipMemsetAsync(L->dPdf, 0, pdfBytes, L->c.stream), "hipMemset")) { list_release(L); return; }
-	pair_plan(&L->pair, L->c.args, L->c.nCU, ld, (uint64_t)L->nCells, true);
+	pair_plan(&L->pair, L->c, ld, (uint64_t)L->nCells, true);
 	L->momentBlocks = (L->nFluid + 255) / 256;
 	if (!dev_alloc((void **)&L->dMoments, sizeof(double) * (2 * (size_t)L->momentBlocks + 2), "moment scratch")) { list_release(L); return; }
 	if (!L->c.args.lazyShadow) {

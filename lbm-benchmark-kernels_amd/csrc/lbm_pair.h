@@ -19,6 +19,7 @@ struct PairPlan {
 	int X = 0, Y = 0, Z = 0, py = 0, pz = 0;
 	int y0 = 0, y1 = 0, z0 = 0, z1 = 0;   // range the tiles cover (solid faces left out)
 	int prec = 0, f16Shift = 0;
+	int device = 0;              // the lattice's, whatever the calling thread's current one is
 	uint64_t plane = 0;          // values per direction plane of the arrays stepped
 	int shape = 0;               // tile shape, see lbm_pair.hip
 	int seg = 0, nSeg = 0, nTy = 0, nTz = 0;
@@ -37,7 +38,7 @@ struct PairPlan {
 // periodic axis); otherwise such a lattice is left to the separate kernels.
 // plane: values per direction plane of the kernel's own array, or 0 to step
 // dense ones.
-void pair_plan(PairPlan * p, const KernelArgs & a, int nCU, const LatticeDesc * ld, uint64_t plane, bool openFaces);
+void pair_plan(PairPlan * p, const Common & c, const LatticeDesc * ld, uint64_t plane, bool openFaces);
 
 // Words of `map`.
 size_t pair_map_cells(const PairPlan & p);

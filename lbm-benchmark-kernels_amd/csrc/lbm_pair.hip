@@ -395,9 +395,12 @@ static double pair_shape(PairPlan * p, int nCU)
 	return best;
 }
 
-void pair_plan(PairPlan * p, const KernelArgs & a, int nCU, const LatticeDesc * ld, uint64_t plane, bool openFaces)
+void pair_plan(PairPlan * p, const Common & common, const LatticeDesc * ld, uint64_t plane, bool openFaces)
 {
+	const KernelArgs & a = common.args;
+	const int nCU = common.nCU;
 	*p = PairPlan();
+	p->device = common.device;
 	const int periodic[3] = {ld->PeriodicX, ld->PeriodicY, ld->PeriodicZ};
 	p->X = ld->Dims[0]; p->Y = ld->Dims[1]; p->Z = ld->Dims[2];
 	p->py = periodic[1]; p->pz = periodic[2];
@@ -471,7 +474,11 @@ void pair_alloc(PairPlan * p)
 	const size_t rows = p->useDense ? aligned(sizeof(uint32_t) * (size_t)p->X * p->Y) : 0;
 	const size_t need = pdf + (p->useDense ? pdf : 0) + map + rows;
 	size_t free = 0, total = 0;
-	if (hipMemGetInfo(&free, &total) != hipSuccess || need > free / 2 || hipMalloc(&p->block, need) != hipSuccess) {
+	int current = 0;
+	bool ok = hipGetDevice(&current) == hipSuccess && (current == p->device || hipSetDevice(p->device) == hipSuccess);
+	ok = ok && hipMemGetInfo(&free, &total) == hipSuccess && need <= free / 2 && hipMalloc(&p->block, need) == hipSuccess;
+	if (current != p->device) (void)hipSetDevice(current);
+	if (!ok) {
 		(void)hipGetLastError();
 		p->block = nullptr;
 		p->use = false;

@@ -104,3 +104,21 @@ def test_list_arrays_are_built_again_after_a_failure(stub, what):
         lines = [line for line in log() if line.startswith("launch")]
         assert "k_list_pair_map" in lines[0] and all("k_pair" in line for line in lines[1:]), lines
     """)
+
+
+@pytest.mark.parametrize("name", ["list-aa-pv-soa", "aa-soa"])
+def test_arrays_are_taken_on_the_lattice_s_device(stub, name):
+    """Kernel() called while another device is current allocates on the
+    device that Init ran on, and leaves the current one as it was."""
+    stub(f"""
+        C.c_int.in_dll(S, "stub_devices").value = 2
+        k = kernel({name!r}, (20, 20, 20), ["-two-step", "on"])
+        S.hipSetDevice(1)
+        k.run(case(4))
+        lines = log()
+        assert any("k_pair" in line for line in lines)
+        assert all(line.endswith(" on 0") for line in lines if line.startswith("malloc")), lines
+        d = C.c_int(-1)
+        S.hipGetDevice(C.byref(d))
+        assert d.value == 1
+    """)
