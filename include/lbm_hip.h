@@ -154,6 +154,18 @@ typedef struct {
 } LbmHipTimings;
 int LbmHipGetTimings(const KernelData * kd, LbmHipTimings * out);
 
+/* Two-step launches (-two-step) of a lattice of either kernel.  Init's report
+ * states the plan; whether its arrays fit is known at the Kernel() call. */
+typedef struct {
+	int planned;           /* 1: Kernel() steps the lattice in pairs where their arrays fit */
+	int launches;          /* two-step launches of the last Kernel() call; 0: every step by itself */
+	int tileY, tileZ;      /* cells of a block's tile */
+	int segments;          /* parts along x */
+	uint64_t bytes;        /* device memory the arrays take: not in LbmHipListDeviceBytes */
+	uint64_t held;         /* what they hold at present (0 or bytes) */
+} LbmHipTwoStep;
+int LbmHipTwoStepInfo(const KernelData * kd, LbmHipTwoStep * out);
+
 /* Enables/disables the per-launch events (off by default, or as set by
  * -launch-events).  With them off only loopMs is measured; with them on the
  * even/odd averages are too, at the cost of an event record between
@@ -304,7 +316,7 @@ int LbmHipBatchGraphStats(LbmHipBatch * b, int * slots, long long * captures, lo
  * computed on the host without touching the device: every allocation
  * Init makes, its temporary buffers included, the run-compressed adjacency
  * at its largest, each rounded up to 2 MiB.  What Kernel() takes for -two-step
- * is not in it.  For admission against a memory budget (the serving loop). */
+ * is not in it (LbmHipTwoStepInfo).  For admission against a memory budget (the serving loop). */
 int LbmHipListDeviceBytes(const LatticeDesc * ld, const Parameters * params, uint64_t * bytes);
 
 /* Copies the device list build to caller buffers, in the reference's

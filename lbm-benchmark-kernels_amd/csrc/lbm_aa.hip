@@ -873,7 +873,9 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 	// or NaN force (whose zero components are NaN) the full force table
 	const bool pairs = A->pair.use && !perLaunch && isfinite(cd->XForce);
 	bool inDense = false;      // the dense array is ahead of the full one
+	A->pair.launches = 0;
 	auto pair = [&](bool fl, bool fs) {
+		++A->pair.launches;
 		if (!A->pair.current) aa_dense_copy(A, true);
 		pair_launch(A->pair, A->pair.dense, A->pair.other, k, ft, fl, force, fs, c.stream);
 		std::swap(A->pair.dense, A->pair.other);
@@ -901,6 +903,7 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 		};
 		A->pair.current = false;   // every replay begins and ends with the full array
 		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, A->dPdf, record)) return false;
+		A->pair.launches = pairs ? steps / 2 : 0;
 		A->pair.current = false;
 		synced = false;
 	}
@@ -968,6 +971,8 @@ Common * aa_common(KernelData * kd)
 {
 	return (kd && kd->Kernel == aa_kernel) ? &as_aa(kd)->c : nullptr;
 }
+
+PairPlan * aa_pair(KernelData * kd) { return aa_common(kd) ? &as_aa(kd)->pair : nullptr; }
 
 bool aa_steps(KernelData * kd, const CaseData * cd)
 {

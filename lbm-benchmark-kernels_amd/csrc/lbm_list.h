@@ -89,6 +89,7 @@ __global__ __launch_bounds__(B) void k_sum_pairs(const double * __restrict__ par
 
 // aa-soa counterparts of the list kernel's moment sums and step runs
 // (lbm_aa.hip): false with the error recorded.
+PairPlan * aa_pair(KernelData * kd);      // null: not an aa-soa kernel
 bool aa_moments(KernelData * kd, double * mass, double * jx);
 bool aa_steps(KernelData * kd, const CaseData * cd);
 bool aa_download_shadow(KernelData * kd);

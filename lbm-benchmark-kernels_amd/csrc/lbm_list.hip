@@ -714,7 +714,9 @@ static bool list_steps(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 	bool pairs = L->pair.use && !perLaunch && isfinite(cd->XForce) && steps > 0;
 	if (pairs && !list_build_pair(L)) return false;
 	pairs = pairs && L->pair.use;
+	L->pair.launches = 0;
 	auto pair = [&](bool fl, bool fs) {
+		++L->pair.launches;
 		pair_launch(L->pair, L->dPdf, L->pair.other, k, ft, fl, force, fs, c.stream);
 		std::swap(L->dPdf, L->pair.other);
 	};
@@ -739,6 +741,7 @@ static bool list_steps(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 			}
 		};
 		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, L->dPdf, record)) return false;
+		L->pair.launches = pairs ? steps / 4 * 2 : 0;
 		synced = false;
 	}
 	for (int it = 0; it < steps && L->nFluid > 0 && !useGraph; it += 2) {
@@ -1202,6 +1205,22 @@ int LbmHipRunSteady(KernelData * kd, CaseData * cd, int checkEvery, double tol, 
 {
 	if (!list_data(kd) && !aa_common(kd)) { fail("LbmHipRunSteady: not a kernel of this library."); return -1; }
 	return run_steady(kd, cd, checkEvery, tol, maxSteps, out, "LbmHipRunSteady");
+}
+
+int LbmHipTwoStepInfo(const KernelData * kd, LbmHipTwoStep * out)
+{
+	KernelData * k = const_cast<KernelData *>(kd);
+	const PairPlan * p = list_data(k) ? &list_data(k)->pair : aa_pair(k);
+	if (!p || !out) { fail("LbmHipTwoStepInfo: not a kernel of this library."); return -1; }
+	*out = LbmHipTwoStep();
+	out->launches = p->launches;
+	if (!p->use) return 0;
+	out->planned = 1;
+	pair_tile(*p, &out->tileY, &out->tileZ);
+	out->segments = p->nSeg;
+	out->bytes = pair_bytes(*p);
+	out->held = p->block ? out->bytes : 0;
+	return 0;
 }
 
 int LbmHipListCopyBuild(const KernelData * kd, uint32_t * adj, uint32_t * grid, uint32_t * coords)

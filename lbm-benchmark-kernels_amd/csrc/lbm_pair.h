@@ -30,6 +30,7 @@ struct PairPlan {
 	uint32_t * rows = nullptr;   // scratch of the dense map: one word per z row
 	bool useDense = false;       // the arrays stepped are dense and other
 	bool current = false;        // dense holds the kernel's present state
+	int launches = 0;            // of the last Kernel() call
 };
 
 // Decides whether the lattice is stepped in pairs (-two-step) and sets the
@@ -42,6 +43,10 @@ void pair_plan(PairPlan * p, const Common & c, const LatticeDesc * ld, uint64_t 
 
 // Words of `map`.
 size_t pair_map_cells(const PairPlan & p);
+// Device memory of all the arrays.
+size_t pair_bytes(const PairPlan & p);
+// Cells of a tile in y and z.
+void pair_tile(const PairPlan & p, int * y, int * z);
 
 // Allocates the arrays of a plan in use that has none yet.  Where they would
 // take more than half of the device's free memory the lattice is left to the

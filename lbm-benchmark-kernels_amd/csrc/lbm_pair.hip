@@ -465,14 +465,28 @@ void pair_report(const PairPlan & p)
 		       kTileZ[p.shape], p.nSeg, p.seg);
 }
 
+void pair_tile(const PairPlan & p, int * y, int * z)
+{
+	*y = kTileY[p.shape];
+	*z = kTileZ[p.shape];
+}
+
+static size_t aligned(size_t n) { return (n + 4095) / 4096 * 4096; }
+static size_t pdf_bytes(const PairPlan & p)
+{
+	return aligned((p.prec == PREC_FP64 ? 8 : p.prec == PREC_FP32S ? 4 : 2) * (size_t)19 * p.plane);
+}
+static size_t row_bytes(const PairPlan & p) { return p.useDense ? aligned(sizeof(uint32_t) * (size_t)p.X * p.Y) : 0; }
+
+size_t pair_bytes(const PairPlan & p)
+{
+	return (p.useDense ? 2 : 1) * pdf_bytes(p) + aligned(sizeof(uint32_t) * pair_map_cells(p)) + row_bytes(p);
+}
+
 void pair_alloc(PairPlan * p)
 {
 	if (!p->use || p->block) return;
-	auto aligned = [](size_t n) { return (n + 4095) / 4096 * 4096; };
-	const size_t pdf = aligned((p->prec == PREC_FP64 ? 8 : p->prec == PREC_FP32S ? 4 : 2) * (size_t)19 * p->plane);
-	const size_t map = aligned(sizeof(uint32_t) * pair_map_cells(*p));
-	const size_t rows = p->useDense ? aligned(sizeof(uint32_t) * (size_t)p->X * p->Y) : 0;
-	const size_t need = pdf + (p->useDense ? pdf : 0) + map + rows;
+	const size_t pdf = pdf_bytes(*p), need = pair_bytes(*p);
 	size_t free = 0, total = 0;
 	int current = 0;
 	bool ok = hipGetDevice(&current) == hipSuccess && (current == p->device || hipSetDevice(p->device) == hipSuccess);
@@ -491,7 +505,7 @@ void pair_alloc(PairPlan * p)
 		p->dense = at;
 		at += pdf;
 		p->rows = (uint32_t *)at;
-		at += rows;
+		at += row_bytes(*p);
 	}
 	p->map = (uint32_t *)at;
 }

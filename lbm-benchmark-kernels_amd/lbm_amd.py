@@ -85,6 +85,11 @@ class LbmHipListInfo(C.Structure):
                 ("nRunsWave", C.c_int), ("adjRle", C.c_int), ("prec", C.c_int)]
 
 
+class LbmHipTwoStep(C.Structure):
+    _fields_ = [("planned", C.c_int), ("launches", C.c_int), ("tileY", C.c_int), ("tileZ", C.c_int),
+                ("segments", C.c_int), ("bytes", C.c_uint64), ("held", C.c_uint64)]
+
+
 class LbmHipSteady(C.Structure):
     _fields_ = [("steps", C.c_int), ("converged", C.c_int), ("relChange", C.c_double),
                 ("mass", C.c_double), ("momentumX", C.c_double), ("seconds", C.c_double)]
@@ -126,7 +131,7 @@ HIP_SYMBOLS = ["D3Q19ListAaPvInit_PushSoAHip", "D3Q19ListAaPvDeinit_PushSoAHip",
                "LbmHipBatchRemove", "LbmHipBatchKernelData", "LbmHipBatchStatusOf", "LbmHipBatchStep",
                "LbmHipBatchRun", "LbmHipBatchSync", "LbmHipBatchGetTuning", "LbmHipBatchSetTuning",
                "LbmHipBatchAutotune", "LbmHipBatchStats", "LbmHipBatchGraphStats", "LbmHipBatchLaunch", "LbmHipBatchWait",
-               "LbmHipListBuildNoAlloc", "LbmHipListDeviceBytes"]
+               "LbmHipListBuildNoAlloc", "LbmHipListDeviceBytes", "LbmHipTwoStepInfo"]
 HOST_SYMBOLS = ["D3Q19_X", "D3Q19_Y", "D3Q19_Z", "D3Q19_INV", "D3Q19_NAMES", "KernelDensity", "VtkWrite",
                 "KernelStatistics", "KernelStatisticsAdv", "KernelSetInitialDensity",
                 "KernelSetInitialVelocity", "KernelVerifiy", "KernelAddBodyForce", "GeoCreateByType",
@@ -185,6 +190,7 @@ def hip_lib() -> C.CDLL:
         L.LbmHipSetShadowDownload.argtypes = [KD, C.c_int]
         L.LbmHipSyncShadow.argtypes = [KD]
         L.LbmHipListGetInfo.argtypes = [KD, C.POINTER(LbmHipListInfo)]
+        L.LbmHipTwoStepInfo.argtypes = [KD, C.POINTER(LbmHipTwoStep)]
         L.LbmHipListCopyBuild.argtypes = [KD, C.c_void_p, C.c_void_p, C.c_void_p]
         L.LbmHipDumpNodes.argtypes = [KD, C.POINTER(LatticeDesc), C.c_void_p]
         L.LbmHipLoadNodes.argtypes = [KD, C.POINTER(LatticeDesc), C.c_void_p]
@@ -413,6 +419,13 @@ class Kernel:
 
     def set_shadow_download(self, on: bool):
         hip_lib().LbmHipSetShadowDownload(self.kd, int(on))
+
+    def two_step(self) -> LbmHipTwoStep:
+        """What the two-step launch does on this lattice (LbmHipTwoStepInfo)."""
+        info = LbmHipTwoStep()
+        if hip_lib().LbmHipTwoStepInfo(self.kd, C.byref(info)) != 0:
+            raise RuntimeError(hip_lib().LbmHipLastError().decode())
+        return info
 
     def list_info(self) -> LbmHipListInfo:
         info = LbmHipListInfo()

@@ -83,6 +83,37 @@ def test_init_reports_a_failed_launch_when_memory_is_short(stub):
     """)
 
 
+@pytest.mark.parametrize("name", ["list-aa-pv-soa", "aa-soa"])
+def test_two_step_info_says_what_the_call_did(stub, name):
+    """LbmHipTwoStepInfo counts the two-step launches that the last call made,
+    also from a replayed graph and where the arrays did not fit."""
+    stub(f"""
+        def check(k, steps, want):
+            log()
+            k.run(case(steps))
+            made = launches("k_pair")
+            assert k.two_step().launches == want, (k.two_step().launches, want)
+            return made
+        name = {name!r}
+        k = kernel(name, (20, 20, 20), ["-two-step", "on"])
+        i = k.two_step()
+        assert i.planned and (i.tileY, i.tileZ, i.segments) == (5, 32, 20) and i.bytes > 0
+        assert check(k, 6, 3) == 3 and k.two_step().held == i.bytes
+        k.set_launch_events(True)
+        assert check(k, 6, 0) == 0
+        k = kernel(name, (20, 20, 20), ["-two-step", "on", "-graph", "on"])
+        want = 2 if name == "list-aa-pv-soa" else 3          # an odd number of pairs: one in place
+        assert check(k, 6, want) == want and check(k, 6, want) == 0
+        k = kernel(name, (20, 20, 20), ["-two-step", "off"])
+        assert not k.two_step().planned and check(k, 6, 0) == 0
+        if name == "list-aa-pv-soa":
+            k = kernel(name, (20, 20, 20), ["-two-step", "on"])
+            free_bytes(i.bytes + 4096)                       # more than half of it
+            assert k.two_step().planned
+            assert check(k, 6, 0) == 0 and k.two_step().held == 0
+    """)
+
+
 @pytest.mark.parametrize("what", ["launch", "memset"])
 def test_list_arrays_are_built_again_after_a_failure(stub, what):
     """A Kernel() call that could not fill the cell map or clear the second
