@@ -87,7 +87,7 @@
  *                     -even-cap, -odd-order, -even-order, -odd-pairs, -vec --
  *                     is given; on: wherever the faces allow it; off).  The
  *                     second array (aa-soa: two) and an index map are taken
- *                     at the first Kernel() call (aa-soa: at Init), only
+ *                     at the first Kernel() call that steps in pairs, only
  *                     where they fit into half of the free device memory;
  *                     otherwise, with -launch-events, with a non-finite body
  *                     force and in a batch the steps are launched one by one

@@ -723,21 +723,31 @@ static void aa_dense_copy(AaData * A, bool toDense)
 	A->pair.current = true;
 }
 
-// The arrays of the two-step launch; the number of fluid cells in the mask to
-// *count (device).  Launches before this call are checked by the caller:
-// pair_alloc leaves no error behind where it takes no memory.
-static bool aa_build_pair(AaData * A, const LatticeDesc * ld, uint32_t * count, hipStream_t s)
+// The arrays of the two-step launch, made at the first call that uses them:
+// a lattice that is never stepped in pairs takes none, and Init no more than
+// the lattice itself.
+static bool aa_build_pair(AaData * A)
 {
-	const AaGeom & g = A->g;
 	PairPlan & p = A->pair;
-	pair_plan(&p, A->c, ld, 0, false);
+	if (!p.use || p.block) return true;
 	pair_alloc(&p);
 	if (!p.use) return true;
+	const AaGeom & g = A->g;
 	const uint32_t rows = (uint32_t)g.X * g.Y;
+	uint32_t * count = p.rows + rows, n = 0;       // fluid cells of the mask
+	hipStream_t s = A->c.stream;
+	(void)hipGetLastError();
 	k_aa_row_counts<<<(rows + 255) / 256, 256, 0, s>>>(A->dFluid, g, p.rows);
 	scan_exclusive(p.rows, rows, count, s);
 	k_aa_pair_map<<<(unsigned)((pair_map_cells(p) + 255) / 256), 256, 0, s>>>(A->dFluid, g, p.rows, p.map);
-	return hip_ok(hipGetLastError(), "cell map kernel");
+	if (!hip_ok(hipGetLastError(), "cell map kernel") ||
+	    !hip_ok(hipMemcpyAsync(&n, count, sizeof(n), hipMemcpyDeviceToHost, s), "count download") ||
+	    !hip_ok(hipStreamSynchronize(s), "cell map kernel")) {
+		pair_release(&p);
+		return false;
+	}
+	if (n != (uint32_t)A->nFluid) pair_free(&p);   // the dense planes are sized by nFluid
+	return true;
 }
 
 // Host copy of the current state for the output functions' GetNode.
@@ -871,7 +881,9 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 
 	// both steps in one launch; per-launch timing needs two, and an infinite
 	// or NaN force (whose zero components are NaN) the full force table
-	const bool pairs = A->pair.use && !perLaunch && isfinite(cd->XForce);
+	bool pairs = A->pair.use && !perLaunch && isfinite(cd->XForce) && steps > 0;
+	if (pairs && !aa_build_pair(A)) return false;
+	pairs = pairs && A->pair.use;
 	bool inDense = false;      // the dense array is ahead of the full one
 	A->pair.launches = 0;
 	auto pair = [&](bool fl, bool fs) {
@@ -1102,24 +1114,23 @@ void D3Q19AaInit_AaSoAHip(LatticeDesc * ld, KernelData ** kernelData, Parameters
 
 	int * dMask = nullptr;
 	uint32_t * dCount = nullptr;
-	uint32_t hCount[2] = {0, 0};     // bounce-back pairs; fluid cells (with a two-step plan)
+	uint32_t hCount = 0;
 	bool ok = false;
 	hipStream_t s = A->c.stream;
 	do {
 		if (!hip_ok(hipMalloc((void **)&dMask, sizeof(int) * nTotal), "allocating geometry mask")) break;
-		if (!hip_ok(hipMalloc((void **)&dCount, sizeof(hCount)), "allocating counter")) break;
+		if (!hip_ok(hipMalloc((void **)&dCount, sizeof(uint32_t)), "allocating counter")) break;
 		if (!hip_ok(hipMalloc((void **)&A->dInfo, sizeof(uint32_t) * nTotal), "allocating cell info")) break;
 		const uint64_t nWords = (uint64_t)g.X * g.Y * g.zWords;
 		if (!hip_ok(hipMalloc((void **)&A->dFluid, sizeof(unsigned long long) * nWords), "allocating fluid mask")) break;
 		if (!hip_ok(hipMalloc((void **)&A->dPdf, aa_bytes(A)), "allocating device lattice")) break;
 		if (!hip_ok(hipMemcpyAsync(dMask, ld->Lattice, sizeof(int) * nTotal, hipMemcpyHostToDevice, s), "mask upload")) break;
-		if (!hip_ok(hipMemsetAsync(dCount, 0, sizeof(hCount), s), "hipMemset")) break;
+		if (!hip_ok(hipMemsetAsync(dCount, 0, sizeof(uint32_t), s), "hipMemset")) break;
 		(void)hipGetLastError();
 		k_aa_info<<<(unsigned)((nTotal + 255) / 256), 256, 0, s>>>(dMask, g, A->dInfo, dCount);
 		k_aa_fluid_bits<<<(unsigned)((nWords + 255) / 256), 256, 0, s>>>(A->dInfo, g, A->dFluid);
 		if (!hip_ok(hipGetLastError(), "cell info kernel")) break;
-		if (!aa_build_pair(A, ld, dCount + 1, s)) break;
-		if (!hip_ok(hipMemcpyAsync(hCount, dCount, sizeof(hCount), hipMemcpyDeviceToHost, s), "count download")) break;
+		if (!hip_ok(hipMemcpyAsync(&hCount, dCount, sizeof(uint32_t), hipMemcpyDeviceToHost, s), "count download")) break;
 		A->hPdf = host_alloc(aa_bytes(A));
 		if (!A->hPdf) { fail("allocating host lattice failed: %zu bytes.", aa_bytes(A)); break; }
 		// every slot starts as f = 0, ghost cells included; shifted storage
@@ -1137,9 +1148,8 @@ void D3Q19AaInit_AaSoAHip(LatticeDesc * ld, KernelData ** kernelData, Parameters
 	(void)hipFree(dMask);
 	(void)hipFree(dCount);
 	if (!ok) { aa_release(A); return; }
-	A->nBounce = (int)hCount[0];
-	// the dense planes are sized by nFluid
-	if (A->pair.use && hCount[1] != (uint32_t)A->nFluid) pair_free(&A->pair);
+	A->nBounce = (int)hCount;
+	pair_plan(&A->pair, A->c, ld, 0, false);
 	if (!A->c.args.quiet) {
 		pair_report(A->pair);
 		printf("# bounce back pdfs: %d (resolved in the odd step, no index lists)\n", A->nBounce);

@@ -27,7 +27,7 @@ struct PairPlan {
 	uint32_t * map = nullptr;
 	void * other = nullptr;
 	void * dense = nullptr;
-	uint32_t * rows = nullptr;   // scratch of the dense map: one word per z row
+	uint32_t * rows = nullptr;   // scratch of the dense map: one word per z row and their sum
 	bool useDense = false;       // the arrays stepped are dense and other
 	bool current = false;        // dense holds the kernel's present state
 	int launches = 0;            // of the last Kernel() call

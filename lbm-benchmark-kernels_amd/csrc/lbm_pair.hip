@@ -476,7 +476,10 @@ static size_t pdf_bytes(const PairPlan & p)
 {
 	return aligned((p.prec == PREC_FP64 ? 8 : p.prec == PREC_FP32S ? 4 : 2) * (size_t)19 * p.plane);
 }
-static size_t row_bytes(const PairPlan & p) { return p.useDense ? aligned(sizeof(uint32_t) * (size_t)p.X * p.Y) : 0; }
+static size_t row_bytes(const PairPlan & p)
+{
+	return p.useDense ? aligned(sizeof(uint32_t) * ((size_t)p.X * p.Y + 1)) : 0;
+}
 
 size_t pair_bytes(const PairPlan & p)
 {

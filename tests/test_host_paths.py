@@ -106,11 +106,31 @@ def test_two_step_info_says_what_the_call_did(stub, name):
         assert check(k, 6, want) == want and check(k, 6, want) == 0
         k = kernel(name, (20, 20, 20), ["-two-step", "off"])
         assert not k.two_step().planned and check(k, 6, 0) == 0
-        if name == "list-aa-pv-soa":
-            k = kernel(name, (20, 20, 20), ["-two-step", "on"])
-            free_bytes(i.bytes + 4096)                       # more than half of it
-            assert k.two_step().planned
-            assert check(k, 6, 0) == 0 and k.two_step().held == 0
+        k = kernel(name, (20, 20, 20), ["-two-step", "on"])
+        free_bytes(i.bytes + 4096)                           # more than half of it
+        assert k.two_step().planned
+        assert check(k, 6, 0) == 0 and k.two_step().held == 0
+    """)
+
+
+def test_aa_init_takes_the_lattice_alone(stub):
+    """aa-soa's Init allocates as much with two-step launches as without, and
+    a lattice stepped with launch events never takes their arrays."""
+    stub("""
+        def taken(mode):
+            before = free_bytes()
+            k = kernel("aa-soa", (20, 20, 20), ["-two-step", mode])
+            return k, before - free_bytes()
+        a, plain = taken("off")
+        b, paired = taken("on")
+        assert paired == plain, (paired, plain)
+        before = free_bytes()
+        b.set_launch_events(True)
+        b.run(case(4))
+        assert free_bytes() == before
+        b.set_launch_events(False)
+        b.run(case(4))
+        assert before - free_bytes() == b.two_step().held == b.two_step().bytes
     """)
 
 
