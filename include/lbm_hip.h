@@ -88,7 +88,8 @@
  *                     is given; on: wherever the faces allow it; off).  The
  *                     second array (aa-soa: two) and an index map are taken
  *                     at the first Kernel() call that steps in pairs, only
- *                     where they fit into half of the free device memory;
+ *                     where they fit into half of the free device memory,
+ *                     and given back when an Init or a batch needs them;
  *                     otherwise, with -launch-events, with a non-finite body
  *                     force and in a batch the steps are launched one by one
  *   -odd-pairs auto|on|off
@@ -165,6 +166,12 @@ typedef struct {
 	uint64_t held;         /* what they hold at present (0 or bytes) */
 } LbmHipTwoStep;
 int LbmHipTwoStepInfo(const KernelData * kd, LbmHipTwoStep * out);
+/* Gives the arrays of a lattice back (kd NULL: of every lattice on the current
+ * device), for a program that needs the memory elsewhere; the lattice keeps
+ * its state, and its next Kernel() call that steps in pairs takes them again.
+ * Arrays that a Kernel() call is using at the moment stay.  The library does
+ * the same by itself when an allocation of its own (Init, a batch) would fail. */
+int LbmHipTwoStepRelease(KernelData * kd);
 
 /* Enables/disables the per-launch events (off by default, or as set by
  * -launch-events).  With them off only loopMs is measured; with them on the

@@ -729,9 +729,7 @@ static void aa_dense_copy(AaData * A, bool toDense)
 static bool aa_build_pair(AaData * A)
 {
 	PairPlan & p = A->pair;
-	if (!p.use || p.block) return true;
-	pair_alloc(&p);
-	if (!p.use) return true;
+	if (p.block || !pair_alloc(&p)) return true;
 	const AaGeom & g = A->g;
 	const uint32_t rows = (uint32_t)g.X * g.Y;
 	uint32_t * count = p.rows + rows, n = 0;       // fluid cells of the mask
@@ -882,8 +880,9 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 	// both steps in one launch; per-launch timing needs two, and an infinite
 	// or NaN force (whose zero components are NaN) the full force table
 	bool pairs = A->pair.use && !perLaunch && isfinite(cd->XForce) && steps > 0;
+	const PairUse use(A->pair.use ? &A->pair : nullptr);
 	if (pairs && !aa_build_pair(A)) return false;
-	pairs = pairs && A->pair.use;
+	pairs = pairs && A->pair.block;
 	bool inDense = false;      // the dense array is ahead of the full one
 	A->pair.launches = 0;
 	auto pair = [&](bool fl, bool fs) {
@@ -914,7 +913,7 @@ static bool aa_run(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 			pairs_done();
 		};
 		A->pair.current = false;   // every replay begins and ends with the full array
-		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, A->dPdf, record)) return false;
+		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, A->dPdf, pairs ? A->pair.generation : 0, record)) return false;
 		A->pair.launches = pairs ? steps / 2 : 0;
 		A->pair.current = false;
 		synced = false;
@@ -1013,7 +1012,7 @@ bool aa_moments(KernelData * kd, double * mass, double * jx)
 	const AaGeom g = A->g;
 	const uint32_t nb = (uint32_t)(((uint64_t)g.X * g.Y * g.Z + 255) / 256);
 	if (!A->dMoments) {
-		if (!hip_ok(hipMalloc((void **)&A->dMoments, sizeof(double) * 2 * ((size_t)nb + 1)), "allocating moment sums")) return false;
+		if (!hip_ok(device_alloc((void **)&A->dMoments, sizeof(double) * 2 * ((size_t)nb + 1)), "allocating moment sums")) return false;
 		A->momentBlocks = nb;
 	}
 	double * part = A->dMoments, * sum = A->dMoments + 2 * (size_t)nb;
@@ -1043,7 +1042,7 @@ static void aa_release(AaData * A)
 	(void)hipFree(A->dInfo);
 	(void)hipFree(A->dFluid);
 	(void)hipFree(A->dPdf);
-	pair_free(&A->pair);
+	pair_release(&A->pair);
 	host_free(A->hPdf);
 	free(A->hInfo);
 	common_free(&A->c);
@@ -1118,12 +1117,12 @@ void D3Q19AaInit_AaSoAHip(LatticeDesc * ld, KernelData ** kernelData, Parameters
 	bool ok = false;
 	hipStream_t s = A->c.stream;
 	do {
-		if (!hip_ok(hipMalloc((void **)&dMask, sizeof(int) * nTotal), "allocating geometry mask")) break;
-		if (!hip_ok(hipMalloc((void **)&dCount, sizeof(uint32_t)), "allocating counter")) break;
-		if (!hip_ok(hipMalloc((void **)&A->dInfo, sizeof(uint32_t) * nTotal), "allocating cell info")) break;
+		if (!hip_ok(device_alloc((void **)&dMask, sizeof(int) * nTotal), "allocating geometry mask")) break;
+		if (!hip_ok(device_alloc((void **)&dCount, sizeof(uint32_t)), "allocating counter")) break;
+		if (!hip_ok(device_alloc((void **)&A->dInfo, sizeof(uint32_t) * nTotal), "allocating cell info")) break;
 		const uint64_t nWords = (uint64_t)g.X * g.Y * g.zWords;
-		if (!hip_ok(hipMalloc((void **)&A->dFluid, sizeof(unsigned long long) * nWords), "allocating fluid mask")) break;
-		if (!hip_ok(hipMalloc((void **)&A->dPdf, aa_bytes(A)), "allocating device lattice")) break;
+		if (!hip_ok(device_alloc((void **)&A->dFluid, sizeof(unsigned long long) * nWords), "allocating fluid mask")) break;
+		if (!hip_ok(device_alloc((void **)&A->dPdf, aa_bytes(A)), "allocating device lattice")) break;
 		if (!hip_ok(hipMemcpyAsync(dMask, ld->Lattice, sizeof(int) * nTotal, hipMemcpyHostToDevice, s), "mask upload")) break;
 		if (!hip_ok(hipMemsetAsync(dCount, 0, sizeof(uint32_t), s), "hipMemset")) break;
 		(void)hipGetLastError();

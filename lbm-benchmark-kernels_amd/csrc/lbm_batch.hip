@@ -287,7 +287,7 @@ static bool grow(void ** p, size_t * capN, size_t needN, size_t elem, const char
 	(void)hipFree(*p);
 	*p = nullptr;
 	const size_t n = needN + needN / 4 + 64;
-	const hipError_t err = hipMalloc(p, n * elem);
+	const hipError_t err = device_alloc(p, n * elem);
 	if (err != hipSuccess) { *capN = 0; return fail("allocating %s failed: %zu bytes (%s).", what, n * elem, hipGetErrorString(err)); }
 	*capN = n;
 	*moved = true;
@@ -421,7 +421,7 @@ static bool rebuild_tables(Batch * b)
 	cap = b->sumCapN;
 	if (!grow((void **)&b->dSums, &cap, sumsN, sizeof(double), "moment sums", &moved)) return false;
 	b->sumCapN = cap;
-	if (!b->dCount && !hip_ok(hipMalloc((void **)&b->dCount, 4 * sizeof(uint32_t)), "allocating chunk counts")) return false;
+	if (!b->dCount && !hip_ok(device_alloc((void **)&b->dCount, 4 * sizeof(uint32_t)), "allocating chunk counts")) return false;
 	if (!b->groups.empty() &&
 	    !grow((void **)&b->dGroupRange, &b->groupCapN, 4 * b->groups.size(), sizeof(uint32_t), "group chunk ranges", &moved))
 		return false;
@@ -1042,7 +1042,7 @@ int LbmHipBatchAutotune(LbmHipBatch * handle, int pairs, LbmHipBatchTuning * out
 		if (x.state != 1) continue;
 		if (!list_upload(x.L)) { release_backup(); return -1; }
 		const size_t bytes = elem_bytes(b->args.prec) * 19 * (size_t)x.L->nCells;
-		if (!hip_ok(hipMalloc(&backup[i], bytes), "allocating the tuning backup") ||
+		if (!hip_ok(device_alloc(&backup[i], bytes), "allocating the tuning backup") ||
 		    !hip_ok(hipMemcpyAsync(backup[i], x.L->dPdf, bytes, hipMemcpyDeviceToDevice, b->stream), "tuning backup")) {
 			release_backup();
 			return -1;

@@ -27,8 +27,7 @@ struct ListData {
 	uint32_t * dGrid = nullptr;
 	uint32_t * dCoords = nullptr;
 	uint32_t * dAdj = nullptr;
-	void * dPdf = nullptr;       // 19 * nCells values of the storage type: dPdfOwn or pair.other
-	void * dPdfOwn = nullptr;
+	void * dPdf = nullptr;       // 19 * nCells values of the storage type
 	PairPlan pair;               // even and odd step in one launch; a launch swaps dPdf and pair.other
 	void * hPdf = nullptr;       // host shadow, same layout and type, == kd.Pdfs[0]
 	double * dMoments = nullptr; // reduction scratch: 2 per block + 2

@@ -463,9 +463,7 @@ __global__ __launch_bounds__(256) void k_list_pair_map(const uint32_t * __restri
 // LbmHipListDeviceBytes states, and a lattice that a batch steps needs none.
 static bool list_build_pair(ListData * L)
 {
-	if (!L->pair.use || L->pair.block) return true;
-	pair_alloc(&L->pair);
-	if (!L->pair.use) return true;
+	if (L->pair.block || !pair_alloc(&L->pair)) return true;
 	(void)hipGetLastError();
 	k_list_pair_map<<<(unsigned)((pair_map_cells(L->pair) + 255) / 256), 256, 0, L->c.stream>>>(
 		L->dGrid, L->dims[0], L->dims[1], L->dims[2], L->periodic[0], L->pair.map);
@@ -712,8 +710,9 @@ static bool list_steps(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 	// both steps in one launch; per-launch timing needs two, and an infinite
 	// or NaN force (whose zero components are NaN) the full force table
 	bool pairs = L->pair.use && !perLaunch && isfinite(cd->XForce) && steps > 0;
+	const PairUse use(L->pair.use ? &L->pair : nullptr);
 	if (pairs && !list_build_pair(L)) return false;
-	pairs = pairs && L->pair.use;
+	pairs = pairs && L->pair.block;
 	L->pair.launches = 0;
 	auto pair = [&](bool fl, bool fs) {
 		++L->pair.launches;
@@ -740,7 +739,7 @@ static bool list_steps(KernelData * kd, const CaseData * cd, LatticeDesc * ld)
 				}
 			}
 		};
-		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, L->dPdf, record)) return false;
+		if (!common_graph_run(&c, steps, cd->Omega, cd->XForce, L->dPdf, pairs ? L->pair.generation : 0, record)) return false;
 		L->pair.launches = pairs ? steps / 4 * 2 : 0;
 		synced = false;
 	}
@@ -842,9 +841,9 @@ static void list_release(ListData * L)
 	(void)hipFree(L->dRunMask);
 	(void)hipFree(L->dRunBase);
 	(void)hipFree(L->dRunAdj);
-	(void)hipFree(L->dPdfOwn);
+	(void)hipFree(L->dPdf);
 	(void)hipFree(L->dMoments);
-	pair_free(&L->pair);
+	pair_release(&L->pair);
 	host_free(L->hPdf);
 	free(L->hGrid);
 	common_free(&L->c);
@@ -854,7 +853,7 @@ static void list_release(ListData * L)
 
 static bool dev_alloc(void ** p, size_t bytes, const char * what)
 {
-	hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+	hipError_t e = device_alloc(p, bytes ? bytes : 1);
 	if (e != hipSuccess) return fail("allocating %s failed: %zu bytes (%s).", what, bytes, hipGetErrorString(e));
 	return true;
 }
@@ -1053,8 +1052,7 @@ void D3Q19ListAaPvInit_PushSoAHip(LatticeDesc * ld, KernelData ** kernelData, Pa
 	// f = w, for FP64 f = 0 as the reference initialises
 	// (src/BenchKernelD3Q19ListAaPvCommon.c:583-585)
 	const size_t pdfBytes = elem_bytes(L->c.args.prec) * 19 * (size_t)L->nCells;
-	if (!dev_alloc((void **)&L->dPdfOwn, pdfBytes, "device lattice")) { list_release(L); return; }
-	L->dPdf = L->dPdfOwn;
+	if (!dev_alloc((void **)&L->dPdf, pdfBytes, "device lattice")) { list_release(L); return; }
 	if (!hip_ok(hipMemsetAsync(L->dPdf, 0, pdfBytes, L->c.stream), "hipMemset")) { list_release(L); return; }
 	pair_plan(&L->pair, L->c, ld, (uint64_t)L->nCells, true);
 	L->momentBlocks = (L->nFluid + 255) / 256;
@@ -1219,7 +1217,21 @@ int LbmHipTwoStepInfo(const KernelData * kd, LbmHipTwoStep * out)
 	pair_tile(*p, &out->tileY, &out->tileZ);
 	out->segments = p->nSeg;
 	out->bytes = pair_bytes(*p);
-	out->held = p->block ? out->bytes : 0;
+	out->held = pair_held(p);
+	return 0;
+}
+
+int LbmHipTwoStepRelease(KernelData * kd)
+{
+	if (!kd) {
+		int device = 0;
+		if (!hip_ok(hipGetDevice(&device), "hipGetDevice")) return -1;
+		(void)pair_reclaim_device(device);
+		return 0;
+	}
+	PairPlan * p = list_data(kd) ? &list_data(kd)->pair : aa_pair(kd);
+	if (!p) { fail("LbmHipTwoStepRelease: not a kernel of this library."); return -1; }
+	(void)pair_reclaim(p);
 	return 0;
 }
 

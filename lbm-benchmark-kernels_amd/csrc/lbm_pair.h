@@ -23,14 +23,18 @@ struct PairPlan {
 	uint64_t plane = 0;          // values per direction plane of the arrays stepped
 	int shape = 0;               // tile shape, see lbm_pair.hip
 	int seg = 0, nSeg = 0, nTy = 0, nTz = 0;
-	void * block = nullptr;      // the allocation that holds all of these
+	void * block = nullptr;      // the allocation of map, rows, dense and dense's other
 	uint32_t * map = nullptr;
-	void * other = nullptr;
+	void * other = nullptr;      // without dense an allocation of its own: it changes places with the kernel's array
 	void * dense = nullptr;
 	uint32_t * rows = nullptr;   // scratch of the dense map: one word per z row and their sum
 	bool useDense = false;       // the arrays stepped are dense and other
 	bool current = false;        // dense holds the kernel's present state
 	int launches = 0;            // of the last Kernel() call
+	unsigned generation = 0;     // counts pair_alloc's allocations: a graph captured with other arrays is stale
+	// arrays that no Kernel() call is using can be given back, see pair_reclaim
+	bool busy = false;
+	PairPlan * next = nullptr;
 };
 
 // Decides whether the lattice is stepped in pairs (-two-step) and sets the
@@ -48,12 +52,29 @@ size_t pair_bytes(const PairPlan & p);
 // Cells of a tile in y and z.
 void pair_tile(const PairPlan & p, int * y, int * z);
 
-// Allocates the arrays of a plan in use that has none yet.  Where they would
-// take more than half of the device's free memory the lattice is left to the
-// separate kernels.
-void pair_alloc(PairPlan * p);
+// Held by a Kernel() call that may step in pairs, from before it looks at the
+// arrays until it returns.
+struct PairUse {
+	PairPlan * p;
+	explicit PairUse(PairPlan * plan);
+	~PairUse();
+	PairUse(const PairUse &) = delete;
+};
+
+// Allocates the arrays unless the plan has them.  False where they would take
+// more than half of the device's free memory: the call goes on with the
+// separate kernels, and a later one asks again.
+bool pair_alloc(PairPlan * p);
 // Frees the arrays; the plan stays, and the next pair_alloc takes them again.
+// Between Kernel() calls they hold nothing that is not in the kernel's own
+// array too, or of use to the next call.
 void pair_release(PairPlan * p);
+// The arrays of one lattice, or of all lattices of a device, given back
+// unless a Kernel() call is using them; the bytes freed.
+size_t pair_reclaim(PairPlan * p);
+size_t pair_reclaim_device(int device);
+// Bytes the arrays hold at present.
+size_t pair_held(const PairPlan * p);
 // The same, and the lattice is stepped by the separate kernels from now on.
 void pair_free(PairPlan * p);
 

@@ -41,6 +41,7 @@
 
 #include <math.h>
 #include <stdio.h>
+#include <mutex>
 
 namespace lbm {
 
@@ -481,43 +482,114 @@ static size_t row_bytes(const PairPlan & p)
 	return p.useDense ? aligned(sizeof(uint32_t) * ((size_t)p.X * p.Y + 1)) : 0;
 }
 
+// Plans that hold arrays, linked through `next`, and their `busy` marks.  The
+// arrays are the library's own choice: an allocation that a lattice cannot do
+// without takes them back from lattices that are not being stepped.
+static std::mutex g_lock;
+static PairPlan * g_held = nullptr;
+
+PairUse::PairUse(PairPlan * plan) : p(plan)
+{
+	if (!p) return;
+	std::lock_guard<std::mutex> hold(g_lock);
+	p->busy = true;
+}
+
+PairUse::~PairUse()
+{
+	if (!p) return;
+	std::lock_guard<std::mutex> hold(g_lock);
+	p->busy = false;
+}
+
 size_t pair_bytes(const PairPlan & p)
 {
 	return (p.useDense ? 2 : 1) * pdf_bytes(p) + aligned(sizeof(uint32_t) * pair_map_cells(p)) + row_bytes(p);
 }
 
-void pair_alloc(PairPlan * p)
+bool pair_alloc(PairPlan * p)
 {
-	if (!p->use || p->block) return;
+	if (p->block) return true;
 	const size_t pdf = pdf_bytes(*p), need = pair_bytes(*p);
 	size_t free = 0, total = 0;
 	int current = 0;
+	void * block = nullptr, * own = nullptr;
 	bool ok = hipGetDevice(&current) == hipSuccess && (current == p->device || hipSetDevice(p->device) == hipSuccess);
-	ok = ok && hipMemGetInfo(&free, &total) == hipSuccess && need <= free / 2 && hipMalloc(&p->block, need) == hipSuccess;
+	ok = ok && hipMemGetInfo(&free, &total) == hipSuccess && need <= free / 2;
+	ok = ok && hipMalloc(&block, need - (p->useDense ? 0 : pdf)) == hipSuccess;
+	ok = ok && (p->useDense || hipMalloc(&own, pdf) == hipSuccess);
 	if (current != p->device) (void)hipSetDevice(current);
 	if (!ok) {
+		(void)hipFree(block);
 		(void)hipGetLastError();
-		p->block = nullptr;
-		p->use = false;
-		return;
+		return false;
 	}
-	char * at = (char *)p->block;
-	p->other = at;
-	at += pdf;
+	char * at = (char *)block;
 	if (p->useDense) {
+		p->other = at;
+		at += pdf;
 		p->dense = at;
 		at += pdf;
 		p->rows = (uint32_t *)at;
 		at += row_bytes(*p);
+	} else {
+		p->other = own;
 	}
 	p->map = (uint32_t *)at;
+	++p->generation;
+	std::lock_guard<std::mutex> hold(g_lock);
+	p->block = block;
+	p->next = g_held;
+	g_held = p;
+	return true;
+}
+
+// With g_lock held.
+static size_t release_locked(PairPlan * p)
+{
+	if (!p->block) return 0;
+	PairPlan ** at = &g_held;
+	while (*at != p) at = &(*at)->next;
+	*at = p->next;
+	p->next = nullptr;
+	(void)hipFree(p->block);
+	if (!p->useDense) (void)hipFree(p->other);
+	p->block = nullptr;
+	p->map = nullptr;
+	p->other = nullptr;
+	p->dense = nullptr;
+	p->rows = nullptr;
+	p->current = false;
+	return pair_bytes(*p);
 }
 
 void pair_release(PairPlan * p)
 {
-	(void)hipFree(p->block);
-	p->block = nullptr;
-	p->current = false;
+	std::lock_guard<std::mutex> hold(g_lock);
+	(void)release_locked(p);
+}
+
+size_t pair_reclaim(PairPlan * p)
+{
+	std::lock_guard<std::mutex> hold(g_lock);
+	return p->busy ? 0 : release_locked(p);
+}
+
+size_t pair_reclaim_device(int device)
+{
+	std::lock_guard<std::mutex> hold(g_lock);
+	size_t freed = 0;
+	for (PairPlan * p = g_held, * next; p; p = next) {
+		next = p->next;
+		if (!p->busy && p->device == device) freed += release_locked(p);
+	}
+	return freed;
+}
+
+size_t pair_held(const PairPlan * p)
+{
+	std::lock_guard<std::mutex> hold(g_lock);
+	return p->block ? pair_bytes(*p) : 0;
 }
 
 void pair_free(PairPlan * p)
@@ -574,6 +646,18 @@ void pair_launch(const PairPlan & p, const void * src, void * dst, const TrtCons
 		case PREC_FP16S: launch_codec(p, src, dst, CodecF16{s16, 1.0f / s16}, k, f, el, ol, fs, stream); break;
 		default: launch_codec(p, src, dst, CodecF64{}, k, f, el, ol, fs, stream);
 	}
+}
+
+// Device memory that the library cannot do without.
+hipError_t device_alloc(void ** p, size_t bytes)
+{
+	hipError_t e = hipMalloc(p, bytes);
+	int device = 0;
+	if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && pair_reclaim_device(device) > 0) {
+		(void)hipGetLastError();
+		e = hipMalloc(p, bytes);
+	}
+	return e;
 }
 
 }  // namespace lbm

@@ -125,6 +125,7 @@ struct Common {
 	int graphSteps = 0;
 	double graphOmega = 0.0, graphForce = 0.0;
 	const void * graphPdf = nullptr;
+	unsigned graphArrays = 0;
 };
 
 // SetNode may change the host shadow only while it holds the device's
@@ -156,14 +157,15 @@ bool common_events(Common * c, int launches);
 void common_collect(Common * c, int launches, bool perLaunch);
 
 // Runs the step loop of `steps` steps for (omega, xForce) on the lattice at
-// `pdf` on c->stream by replaying a HIP graph; `record` issues the loop's kernel launches and is
-// called, under stream capture, only when no graph was captured for these
-// values yet.  The graph holds kernel launches only.
+// `pdf` on c->stream by replaying a HIP graph; `record` issues the loop's
+// kernel launches and is called, under stream capture, only when no graph was
+// captured for these values yet.  The graph holds kernel launches only.
+// arrays: generation of the two-step launch's arrays, 0 for separate launches.
 template <class F>
-bool common_graph_run(Common * c, int steps, double omega, double xForce, const void * pdf, F record)
+bool common_graph_run(Common * c, int steps, double omega, double xForce, const void * pdf, unsigned arrays, F record)
 {
 	if (!c->graphExec || c->graphSteps != steps || c->graphOmega != omega || c->graphForce != xForce ||
-	    c->graphPdf != pdf) {
+	    c->graphPdf != pdf || c->graphArrays != arrays) {
 		common_graph_drop(c);
 		(void)hipGetLastError();
 		if (!hip_ok(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture")) return false;
@@ -182,10 +184,15 @@ bool common_graph_run(Common * c, int steps, double omega, double xForce, const 
 		c->graphOmega = omega;
 		c->graphForce = xForce;
 		c->graphPdf = pdf;
+		c->graphArrays = arrays;
 	}
 	return hip_ok(hipGraphLaunch(c->graphExec, c->stream), "hipGraphLaunch");
 }
 
+// hipMalloc on the current device; when memory is short, lattices that are not
+// being stepped give back the arrays of their two-step launches first.  The
+// caller has checked its launches: a refused allocation clears their error.
+hipError_t device_alloc(void ** p, size_t bytes);
 // Pinned host buffer (hipHostMalloc) -- used for the host shadow.
 void * host_alloc(size_t bytes);
 void host_free(void * p);

@@ -606,8 +606,8 @@ extern "C" int LbmHipStreamBench(uint64_t nDoubles, uint32_t nNodes, int reps, L
 	int rc = -1;
 	do {
 		const size_t bytesA = sizeof(double) * (size_t)(nDoubles > 19ull * nNodes ? nDoubles : 19ull * nNodes);
-		if (!hip_ok(hipMalloc((void **)&a, bytesA), "hipMalloc")) break;
-		if (!hip_ok(hipMalloc((void **)&b, sizeof(double) * (size_t)nDoubles), "hipMalloc")) break;
+		if (!hip_ok(device_alloc((void **)&a, bytesA), "hipMalloc")) break;
+		if (!hip_ok(device_alloc((void **)&b, sizeof(double) * (size_t)nDoubles), "hipMalloc")) break;
 		if (!hip_ok(hipMemset(a, 0, bytesA), "hipMemset")) break;
 		if (!hip_ok(hipEventCreate(&e0), "hipEventCreate") || !hip_ok(hipEventCreate(&e1), "hipEventCreate")) break;
 		const unsigned gc = (unsigned)((nDoubles + 255) / 256), gu = (nNodes + 255) / 256;

@@ -131,7 +131,8 @@ HIP_SYMBOLS = ["D3Q19ListAaPvInit_PushSoAHip", "D3Q19ListAaPvDeinit_PushSoAHip",
                "LbmHipBatchRemove", "LbmHipBatchKernelData", "LbmHipBatchStatusOf", "LbmHipBatchStep",
                "LbmHipBatchRun", "LbmHipBatchSync", "LbmHipBatchGetTuning", "LbmHipBatchSetTuning",
                "LbmHipBatchAutotune", "LbmHipBatchStats", "LbmHipBatchGraphStats", "LbmHipBatchLaunch", "LbmHipBatchWait",
-               "LbmHipListBuildNoAlloc", "LbmHipListDeviceBytes", "LbmHipTwoStepInfo"]
+               "LbmHipListBuildNoAlloc", "LbmHipListDeviceBytes", "LbmHipTwoStepInfo",
+               "LbmHipTwoStepRelease"]
 HOST_SYMBOLS = ["D3Q19_X", "D3Q19_Y", "D3Q19_Z", "D3Q19_INV", "D3Q19_NAMES", "KernelDensity", "VtkWrite",
                 "KernelStatistics", "KernelStatisticsAdv", "KernelSetInitialDensity",
                 "KernelSetInitialVelocity", "KernelVerifiy", "KernelAddBodyForce", "GeoCreateByType",
@@ -191,6 +192,7 @@ def hip_lib() -> C.CDLL:
         L.LbmHipSyncShadow.argtypes = [KD]
         L.LbmHipListGetInfo.argtypes = [KD, C.POINTER(LbmHipListInfo)]
         L.LbmHipTwoStepInfo.argtypes = [KD, C.POINTER(LbmHipTwoStep)]
+        L.LbmHipTwoStepRelease.argtypes = [KD]
         L.LbmHipListCopyBuild.argtypes = [KD, C.c_void_p, C.c_void_p, C.c_void_p]
         L.LbmHipDumpNodes.argtypes = [KD, C.POINTER(LatticeDesc), C.c_void_p]
         L.LbmHipLoadNodes.argtypes = [KD, C.POINTER(LatticeDesc), C.c_void_p]
@@ -426,6 +428,11 @@ class Kernel:
         if hip_lib().LbmHipTwoStepInfo(self.kd, C.byref(info)) != 0:
             raise RuntimeError(hip_lib().LbmHipLastError().decode())
         return info
+
+    def release_two_step(self):
+        """Gives back the device memory of the two-step launch (LbmHipTwoStepRelease)."""
+        if hip_lib().LbmHipTwoStepRelease(self.kd) != 0:
+            raise RuntimeError(hip_lib().LbmHipLastError().decode())
 
     def list_info(self) -> LbmHipListInfo:
         info = LbmHipListInfo()

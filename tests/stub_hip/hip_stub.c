@@ -23,6 +23,8 @@ int stub_devices = 1;
 char stub_fail_launch[128] = "";        /* launches of kernels with this in their name fail */
 char stub_fail_call[64] = "";           /* so does this runtime call ("memset") */
 
+void (*stub_hook)(void) = NULL;         /* called by every hipStreamSynchronize */
+
 static pthread_mutex_t g_lock = PTHREAD_MUTEX_INITIALIZER;
 static char g_log[1 << 22];
 static size_t g_logLen = 0;
@@ -185,7 +187,7 @@ hipError_t hipMemset(void * d, int v, size_t n) { return hipMemsetAsync(d, v, n,
 /* ---- streams, events, graphs ---------------------------------------------- */
 hipError_t hipStreamCreateWithFlags(hipStream_t * s, unsigned f) { (void)f; *s = (hipStream_t)calloc(1, 8); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; if (stub_hook) stub_hook(); return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t * e) { *e = (hipEvent_t)calloc(1, 8); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t * e, unsigned f) { (void)f; return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }

@@ -113,3 +113,26 @@ def test_mixed_with_separate_launches(lbm, name, prec):
     for nodes, moments in out[:2]:
         assert np.array_equal(nodes, out[2][0])
         assert moments == out[2][1]
+
+
+@pytest.mark.parametrize("graph", ["off", "on"])
+@pytest.mark.parametrize("name", ["list-aa-pv-soa", "aa-soa"])
+def test_arrays_given_back_between_calls(lbm, oracle, name, graph):
+    """Calls before and after the arrays were given back, with SetNode between
+    two of them, end in the oracle's state."""
+    dims, per = (17, 15, 35), WALLS
+    mask = _mask(dims, per, 5)
+    geo = lbm.Geometry.from_mask(mask, dims, per)
+    with lbm.Kernel(name, geo, ["-lambda", repr(LAM), "-two-step", "on", "-graph", graph, "-quiet"]) as k:
+        k.set_initial_weights()
+        for call in range(4):
+            k.run(lbm.case_data(omega=1.3, xforce=1e-4, iterations=6))
+            info = k.two_step()
+            assert info.held == info.bytes > 0 and info.launches >= 2
+            if call != 1:
+                k.release_two_step()
+                assert k.two_step().held == 0
+            if call == 2:
+                k.load(k.dump())
+        run = oracle.list_run if name == "list-aa-pv-soa" else oracle.aa_run
+        assert np.array_equal(k.dump(), run(mask, dims, per, 24, 1.3, 1e-4, magic=LAM, force_on=True)[0])

@@ -134,6 +134,63 @@ def test_aa_init_takes_the_lattice_alone(stub):
     """)
 
 
+@pytest.mark.parametrize("name", ["list-aa-pv-soa", "aa-soa"])
+def test_arrays_are_given_back_to_another_lattice(stub, name):
+    """A lattice whose Init fits only without the two-step arrays of another
+    one gets their memory; the other goes on with the separate launches and
+    takes the arrays again once there is room."""
+    stub(f"""
+        a = kernel({name!r}, (40, 40, 40), ["-two-step", "on"])
+        a.run(case(4))
+        held = a.two_step().held
+        assert held > 0
+        free_bytes(held // (2 if {name!r} == "list-aa-pv-soa" else 8))
+        b = kernel({name!r}, (40, 40, 40), ["-two-step", "off"])
+        assert a.two_step().held == 0 and a.two_step().planned
+        log()
+        a.run(case(4))
+        assert a.two_step().launches == 0 and launches("k_pair") == 0
+        b.close()
+        free_bytes(1 << 40)
+        a.run(case(4))
+        assert a.two_step().launches == 2 and a.two_step().held == held and launches("pair_map") == 1
+        a.release_two_step()
+        assert a.two_step().held == 0
+        a.close()
+        c = kernel({name!r}, (40, 40, 40), ["-two-step", "on"])
+        d = kernel({name!r}, (40, 40, 40), ["-two-step", "on"])
+        c.run(case(4)), d.run(case(4))
+        assert lbm.hip_lib().LbmHipTwoStepRelease(None) == 0
+        assert c.two_step().held == d.two_step().held == 0
+        c.run(case(4)), c.close(), d.close()
+    """)
+
+
+@pytest.mark.parametrize("name", ["list-aa-pv-soa", "aa-soa"])
+def test_arrays_in_use_stay_and_graphs_follow_them(stub, name):
+    """Arrays that a Kernel() call is using are not given back, and a graph
+    captured with arrays that were given back is captured anew."""
+    stub(f"""
+        name = {name!r}
+        k = kernel(name, (20, 20, 20), ["-two-step", "on"])
+        HOOK = C.CFUNCTYPE(None)
+        hook = HOOK(lambda: lbm.hip_lib().LbmHipTwoStepRelease(None) and None)
+        C.c_void_p.in_dll(S, "stub_hook").value = C.cast(hook, C.c_void_p).value
+        k.run(case(8))
+        C.c_void_p.in_dll(S, "stub_hook").value = None
+        assert k.two_step().launches == 4 and k.two_step().held > 0
+        k = kernel(name, (20, 20, 20), ["-two-step", "on", "-graph", "on"])
+        for release, captures in ((False, 1), (False, 0), (True, 1), (False, 0)):
+            if release:
+                k.release_two_step()
+            log()
+            k.run(case(8))
+            lines = log()
+            assert lines.count("graph capture") == captures and lines.count("graph replay") == 1, lines
+            assert k.two_step().launches == 4
+    """)
+
+
 @pytest.mark.parametrize("what", ["launch", "memset"])
 def test_list_arrays_are_built_again_after_a_failure(stub, what):
     """A Kernel() call that could not fill the cell map or clear the second
