@@ -372,9 +372,10 @@ static double pair_shape(PairPlan * p, int nCU)
 		const ShapeCost & w = kShapeCost[p->prec][s];
 		if (w.blocksPerCU == 0) continue;
 		const int nTy = (p->y1 - p->y0 + kTileY[s] - 1) / kTileY[s], nTz = (p->z1 - p->z0 + kTileZ[s] - 1) / kTileZ[s];
-		for (int n = 1; n <= p->X; ++n) {
-			const int seg = (p->X + n - 1) / n;
-			if ((p->X + seg - 1) / seg != n) continue;    // the same segments as a smaller n
+		// the distinct segment lengths, each with the smallest n that gives it:
+		// about 2 sqrt(X) of them, a long lattice has far more n
+		for (int n = 1, seg; n <= p->X; n = seg > 1 ? (p->X + seg - 2) / (seg - 1) : p->X + 1) {
+			seg = (p->X + n - 1) / n;
 			const double blocks = (double)nTy * nTz * n, r = blocks / ((double)w.blocksPerCU * nCU);
 			const double rounds = r <= 1.0 ? 1.0 : c.spread * r + (1.0 - c.spread) * ceil(r);
 			const double idle = r <= 1.0 ? 1.0 : rounds / r;

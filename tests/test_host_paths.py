@@ -230,3 +230,23 @@ def test_arrays_are_taken_on_the_lattice_s_device(stub, name):
         S.hipGetDevice(C.byref(d))
         assert d.value == 1
     """)
+
+
+def test_plan_of_a_long_lattice_takes_no_time(stub):
+    """Init's search for segments visits their distinct lengths alone: along
+    8 million cells that is within the noise of Init, where a visit of every
+    number of segments took 150 ms."""
+    stub("""
+        import time
+        import numpy as np
+        X = 8000000
+        g = lbm.Geometry.from_mask(np.ones(X, dtype=np.int32), (X, 1, 1), (0, 0, 0))
+        C.c_uint32.in_dll(S, "stub_count").value = X
+        best = {"off": 1e9, "on": 1e9}
+        for mode in ("off", "on") * 3:
+            t = time.process_time()
+            with lbm.Kernel("list-aa-pv-soa", g, ["-quiet", "-shadow", "lazy", "-prec", "fp16s", "-two-step", mode]) as k:
+                best[mode] = min(best[mode], time.process_time() - t)
+                assert k.two_step().segments == (1024 if mode == "on" else 0)
+        assert best["on"] - best["off"] < 0.075, best
+    """)
