@@ -90,8 +90,12 @@ inline ForceT<R> force_cast(const ForceTerms & t)
 // The reference halves the sum and the difference of an opposite pair before
 // it subtracts the equilibrium; here they are kept whole, the equilibrium is
 // doubled through its constants and the relaxation rates are halved.  Scaling
-// by two commutes with the rounding of every operation, so the results are
-// the same bits, with 19 multiplications fewer per node.
+// by two commutes with the rounding of every operation whose result is
+// normal, so the results are the same bits, with 19 multiplications fewer per
+// node.  Where an intermediate is subnormal (FP32 deviations far ahead of a
+// disturbance) the last bit may differ: halving rounds there once more, so
+// with subnormal values this form lies within 2 of the smallest subnormals
+// of the exact result and the halved one within 5.
 template <class R>
 __device__ __forceinline__ void trt_collide(R (&f)[19], const TrtC<R> & k)
 {
