@@ -30,8 +30,9 @@ int32 adjacency entries = 376 B (doc/main.rst:347), the adjacency compression
 not credited; "moved" counts the bytes the odd kernel needs with the
 run-compressed adjacency (304 B plus 72 B per run and 12 B per 64-node
 wavefront, reported by the library: 317.8 B here).  Where the library does not
-launch pairs (-two-step off, FP16 here) the odd launch is the roofline's kernel.
-step_average_gbs rates the timed steps on the list-AA balance.  The copy and
+launch pairs (-two-step off, FP16 here) the odd launch is the roofline's kernel,
+and step_average_gbs rates the timed steps on the list-AA balance; a pair moves
+less than that balance, so beside k_pair there is no such figure.  The copy and
 update-19 bandwidths of the device are measured in the same run as yardsticks
 (the reference rates its kernels against update-19 bandwidth).
 
@@ -594,6 +595,7 @@ def main():
     b_pair = b_even + 4                         # PDFs in and out, index map
     pair_gbs = b_pair * nf / (2 * loop_s / steps) / 1e9
     even_gbs = b_even * nf / (te.evenMsAvg / 1e3) / 1e9
+    step_gbs = (b_even + b_odd) / 2 * nf * steps / loop_s / 1e9
     print(f"bench: {value:.1f} MFLUP/s loop {t.loopMs:.2f} ms wall {wall * 1e3:.2f} ms even {te.evenMsAvg:.4f} ms "
           f"({even_gbs:.0f} GB/s) odd {te.oddMsAvg:.4f} ms ({odd_gbs:.0f} GB/s at {b_odd} B, {moved_gbs:.0f} GB/s "
           f"at {b_moved:.1f} B) runs={info.nRuns}", file=sys.stderr, flush=True)
@@ -649,7 +651,8 @@ def main():
         "roofline": {"bound": "hbm",
                      "kernel": "k_pair (an even and an odd AA step in one launch)" if pairs else
                                "k_list_odd (odd AA step, run-compressed adjacency)",
-                     "scope": "frac is the named kernel's; step_average_frac is the whole step's on the list-AA balance",
+                     "scope": "frac is the named kernel's" +
+                              ("" if pairs else "; step_average_frac is the whole step's on the list-AA balance"),
                      "achieved": round(pair_gbs if pairs else odd_gbs, 1), "peak": PEAK_GBS, "unit": "GB/s",
                      "frac": round((pair_gbs if pairs else odd_gbs) / PEAK_GBS, 4), "traffic": traffic,
                      "traffic_source": os.path.relpath(traffic_file, ROOT) if traffic is not None else None,
@@ -659,8 +662,8 @@ def main():
                                     "list-AA odd balance: 19 loads + 19 stores + 18 int32 adjacency entries per "
                                     "node, adjacency compression not credited",
                      "ms_avg": 2 * t.loopMs / steps if pairs else te.oddMsAvg,
-                     "step_average_gbs": round((b_even + b_odd) / 2 * nf * steps / loop_s / 1e9, 1),
-                     "step_average_frac": round((b_even + b_odd) / 2 * nf * steps / loop_s / 1e9 / PEAK_GBS, 4),
+                     **({} if pairs else {"step_average_gbs": round(step_gbs, 1),
+                                          "step_average_frac": round(step_gbs / PEAK_GBS, 4)}),
                      "yardsticks_gbs": {"copy": round(yard["copy_gbs"], 1), "update19": round(yard["update19_gbs"], 1)}},
         "separate_launches": {"odd_ms_avg": te.oddMsAvg, "even_ms_avg": te.evenMsAvg,
                               "mflups": round(nf * cd.MaxIterations / (te.loopMs / 1e3) / 1e6, 2),
