@@ -136,3 +136,32 @@ def test_arrays_given_back_between_calls(lbm, oracle, name, graph):
                 k.load(k.dump())
         run = oracle.list_run if name == "list-aa-pv-soa" else oracle.aa_run
         assert np.array_equal(k.dump(), run(mask, dims, per, 24, 1.3, 1e-4, magic=LAM, force_on=True)[0])
+
+
+@pytest.mark.parametrize("prec,plane", [("fp64", 76_695_840), ("fp32s", 153_391_680), ("fp16s", 226_050_896)])
+def test_offsets_up_to_the_window(lbm, oracle, prec, plane):
+    """Direction planes as far apart as the launch takes them (the list
+    kernel's padding): a store reaches up to six planes behind the window's
+    base, 3.7 GB in FP64 and FP32 and 2.7 GB in FP16, where 2^32 PDFs end the
+    range.  One padding step further the steps are launched one by one, with
+    the same results."""
+    dims, per = (17, 15, 35), WALLS
+    mask = _mask(dims, per, 5)
+    geo = lbm.Geometry.from_mask(mask, dims, per)
+    want = _oracle(oracle, "list-aa-pv-soa", mask, dims, per, prec, 1.3, 1e-4)
+    elem = {"fp64": 8, "fp32s": 4, "fp16s": 2}[prec]
+    assert 6 * plane * elem > 2**31 and 19 * plane < 2**32
+    for n in (plane, plane + 16):
+        over = 7 * n * elem > 0xfffffff0
+        if 19 * n > 2**32 - 1:
+            continue
+        print(f"list {prec} planes of {n} values", flush=True)
+        with lbm.Kernel("list-aa-pv-soa", geo, ["-lambda", repr(LAM), "-prec", prec, "-two-step", "on", "-quiet",
+                                                "-shadow", "lazy", "-pad", f"{8 * n}+0"]) as k:
+            assert k.list_info().nCells == n
+            assert lbm.hip_lib().LbmHipSyncShadow(k.kd) == 0
+            k.set_initial_weights()
+            for steps in RUNS:
+                k.run(lbm.case_data(omega=1.3, xforce=1e-4, iterations=steps))
+                assert k.two_step().launches == (0 if over else steps // 2)
+            assert np.array_equal(k.dump(), want), (prec, n)
