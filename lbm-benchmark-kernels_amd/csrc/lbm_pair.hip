@@ -311,9 +311,9 @@ __global__ __launch_bounds__(NT, WAVES) void k_pair(const typename Codec::S * __
 // registers and LDS: at most 512 cells with halo in FP64, 1024 in the narrow
 // types.  Rows of 32 cells and more keep whole lines in a row's accesses;
 // 256^3 FP64 1.20 ms with 13 x 32, 1.33 with 10 x 40, 1.27 with 8 x 48, 1.35
-// with 17 x 24.  The other shapes fit ragged planes (18 x 48, 28 x 32: pipe
-// 129x83x110 FP16 39.5 against 40.7 us and more), small ones (5 x 32: 24^3 7.0
-// against 9.2 us) and large narrow ones (13 x 64).
+// with 17 x 24.  The other shapes fit ragged planes (18 x 48, 28 x 32: measured
+// on one, pipe 129x83x110 FP16, 39.5 against 40.7 us and more), small ones
+// (5 x 32: 24^3 7.0 against 9.2 us) and large narrow ones (13 x 64).
 constexpr int kShapes = 5;
 constexpr int kTileY[kShapes] = {13, 13, 5, 18, 28}, kTileZ[kShapes] = {32, 64, 32, 48, 32};
 constexpr int kTileThreads[kShapes] = {512, 1024, 256, 1024, 1024};
@@ -449,9 +449,12 @@ void pair_plan(PairPlan * p, const Common & common, const LatticeDesc * ld, uint
 	// every cell: 1.04-2.5 in all types, also at 0.55.
 	// Where the separate launches' array fits well into the 256 MiB last-level
 	// cache and two arrays hardly do, the launch reads more from memory than they
-	// do.  At 102 to 187 MiB: FP32 0.81-1.0 and FP64 0.86-1.05 where the
-	// estimates are within a factor of 1.45, 1.0-1.15 where they are further
-	// apart; 1.03-1.29 in both types from 188 MiB on.
+	// do.  Porous media of 102 to 187 MiB, two launches' time over one's: where
+	// the estimates are within a factor of 1.45, FP64 0.86-1.14 and FP32 0.81-1.1
+	// (once 1.37, 126x96x139 at 104 MiB), further apart FP64 0.97-1.2 and FP32
+	// 0.98-1.14.  So what is taken loses 3 % at most, and twelve refused ones would
+	// have gained 5 % on average.  From 188 MiB on 1.03-1.29 in both types.  One
+	// lattice at other addresses varied by 0.94-1.12 (FP64 133x129x75, 172 MiB).
 	double t = pair_shape(p, nCU > 0 ? nCU : 256);
 	const TypeCost & c = kTypeCost[p->prec];
 	const double bytes = 19.0 * (double)elem * ld->nFluid, cache = 256.0 * (1 << 20);
